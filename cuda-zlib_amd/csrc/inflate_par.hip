@@ -20,8 +20,8 @@
 //   emit       one 256-lane workgroup per accepted segment decodes its slices
 //              in parallel, writing output in place; a byte copied from
 //              before its slice's start is marked unresolved with its root
-//   resolve    rounds over the unresolved bitmask, each following up to 32
-//              root links per byte
+//   resolve    the output in stripes, each walked by one workgroup with its last
+//              32 KiB in LDS, then the bytes rooted before their stripe
 //   adler      vectorised Adler-32 partials, then the final status
 //
 // Status semantics restate the reference's general route: framing
@@ -55,7 +55,7 @@ struct State {
   u64 accepted;      // number of accepted segments
   u32 emit_status;
   u32 pad;
-  u64 unresolved[2]; // unresolved bytes after emission / after the last resolve round
+  u64 unresolved;    // unresolved bytes after emission
   u64 recs_used;     // block records handed out by describe
   u64 groups_used;   // 64-slot slice groups handed out by describe
   u64 precount;      // entries of the dense pre-candidate array
@@ -636,7 +636,7 @@ __device__ u32 gzip_fields_group(const u8* in, u64 size, u64 p, Frame& f, u64& z
 // dictionary's Adler-32 against its DICTID (the workgroup sums the bytes).
 // Every workgroup also zeroes its grid-stride share of zero[0..zero_words):
 // the scratch that later kernels accumulate into (Adler-32 pairs, resolve
-// counts, the first unresolved bitmap).
+// count, the unresolved bitmap and its marks).
 __global__ __launch_bounds__(256) void g_frame(const u8* in, u64 in_size, u32 format,
                                                const u8* dict, u64 dict_len, u64 body_off,
                                                u64 out_base, State* st, u32* zero,
@@ -698,8 +698,7 @@ __global__ __launch_bounds__(256) void g_frame(const u8* in, u64 in_size, u32 fo
   st->seeds = 0;
   st->accepted = 0;
   st->emit_status = 0;
-  st->unresolved[0] = 0;
-  st->unresolved[1] = 0;
+  st->unresolved = 0;
   st->recs_used = 0;
   st->groups_used = 0;
   st->precount = 0;
@@ -3544,7 +3543,7 @@ __device__ __forceinline__ bool bit_get(const u32* bits, u64 i) {
 }
 // Resolve groups: the 2048 output bytes of 64 bitmap words, one resolve wave's
 // share.  A byte per group marks a group that may hold unresolved bytes;
-// resolve rounds skip the others.
+// the resolve kernels skip the others.
 constexpr u32 kResolveGroupShift = 11;
 __device__ __forceinline__ void mark_groups(u8* marks, u64 first, u64 n) {
   if (!marks || !n) return;
@@ -3695,7 +3694,7 @@ __global__ __launch_bounds__(64) void g_emit_serial(const u8* body, u64 len, Sta
           for (u32 j = 0; j < length; ++j) {
             const u64 src = dst - distance + (j % distance);
             if (copy_byte(out, roots, unres, seg.prefix, dst + j, src, as, aw, out_end)) {
-              atomicAdd(reinterpret_cast<unsigned long long*>(&st->unresolved[0]), 1ull);
+              atomicAdd(reinterpret_cast<unsigned long long*>(&st->unresolved), 1ull);
               mark_groups(marks, dst + j, 1);
             }
           }
@@ -3719,7 +3718,7 @@ __global__ __launch_bounds__(64) void g_emit_serial(const u8* body, u64 len, Sta
           if (queued) mark_groups(marks, begin + j, 1);
           const u64 bal = __ballot(queued);
           if (!lane && bal)
-            atomicAdd(reinterpret_cast<unsigned long long*>(&st->unresolved[0]), u64(__popcll(bal)));
+            atomicAdd(reinterpret_cast<unsigned long long*>(&st->unresolved), u64(__popcll(bal)));
         }
       } else {
         for (u64 j = lane; j < length; j += kWave) {
@@ -3809,7 +3808,7 @@ __device__ __forceinline__ void bits_set_range(u32* bits, u64 start, u32 n) {
 // with kAdler adds every byte to the thread's Adler-32 sums); StagedBytes
 // writes a workgroup's LDS stage that holds output positions [base, ...),
 // copied out (and summed) once the round is done.  zero() fills bytes whose
-// value a later resolve round provides.
+// value resolution provides later.
 template <bool kAdler>
 struct GlobalBytes {
   u8* out;
@@ -3840,7 +3839,7 @@ struct StagedBytes {
 // (copied out and summed when the round is done), later ones straight to
 // the output buffer (summed as they are written).  The stage is all zero
 // when a round starts (the copy-out clears what it read), so the bytes a
-// resolve round provides are zero without a store each.
+// resolution provides are zero without a store each.
 // Byte pointers into LDS and into global memory, typed with their address
 // spaces so that the compiler issues LDS or global instructions: a flat one
 // (what a pointer chosen between the two becomes) counts against both wait
@@ -4011,7 +4010,7 @@ __device__ __forceinline__ void emit_match(const Sink& out, u64 dst0, u64 dst, u
       // output is rooted at its source without checking whether that is
       // resolved: a load of the bitmap (or of the source's root) here would
       // wait for every store the wave has pending.  A resolved source only
-      // costs the resolve rounds one link.
+      // costs resolution one link.
       if (src < dst0 || nunres) {
         roots[d] = last = u32(src);
         bit_set(unres, d);
@@ -4421,7 +4420,7 @@ __global__ __launch_bounds__(kEmitThreads) __attribute__((amdgpu_waves_per_eu(4)
   }
   for (u32 off = 32; off; off >>= 1) unres_total += __shfl_down(unres_total, off, 64);
   if (lane_id() == 0 && unres_total)
-    atomicAdd(reinterpret_cast<unsigned long long*>(&st->unresolved[0]), unres_total);
+    atomicAdd(reinterpret_cast<unsigned long long*>(&st->unresolved), unres_total);
   // The workgroup's Adler-32 partial pair.
   u64 ps = sums.s % kAdlerMod, pw = sums.w % kAdlerMod;
   for (u32 off = 32; off; off >>= 1) {
@@ -4450,14 +4449,14 @@ __global__ __launch_bounds__(kEmitThreads) __attribute__((amdgpu_waves_per_eu(4)
 // Large files of a batch: one 256-thread workgroup per file decodes its
 // blocks in turn: a stored block by a copy, a fixed or dynamic block by
 // describe's parallel slices and then one slice per thread, as g_emit_lanes
-// does.  Copies that reach before their slice are left to g_resolve over the
+// does.  Copies that reach before their slice are left to resolution over the
 // batch output.  A file whose decode meets anything unusual (any status, an
 // exhausted slice-group pool, a bad encoded row) is flagged in `redo` for
 // the serial per-file decoder, which restates the reference's statuses.
 __global__ __launch_bounds__(kDescThreads) void g_batch_wide(
     const u8* in, u8* out, const BatchFile* files, const u32* list, u32 n, const u32* encoded,
     u32 max_blocks, State* st, u64* slice_entry, u32* slice_off, u32* group_link,
-    u64 group_capacity, u32* roots, u32* unres, u32* redo, u32* wanted) {
+    u64 group_capacity, u32* roots, u32* unres, u32* redo, u32* wanted, u8* marks) {
   __shared__ DescShared sh;
   __shared__ u64 e_first, e_chunk_end;
   __shared__ u32 e_count, e_next, e_need, bad, window;
@@ -4551,12 +4550,12 @@ __global__ __launch_bounds__(kDescThreads) void g_batch_wide(
               lerr = emit_slice<false, false>(sh, blim, e_rel, s_rel, dst0, block_end, window,
                                        GlobalBytes<false>{out, nullptr, 0}, roots,
                                        unres, unres_total, base, false, no_lead, no_last,
-                                       nullptr);
+                                       marks);
             else
               lerr = emit_slice<true, false>(sh, blim, e_rel, s_rel, dst0, block_end, window,
                                       GlobalBytes<false>{out, nullptr, 0}, roots,
                                       unres, unres_total, base, false, no_lead, no_last,
-                                      nullptr);
+                                      marks);
             if (lerr) bad = 1;
           }
           done += count;
@@ -4580,7 +4579,7 @@ __global__ __launch_bounds__(kDescThreads) void g_batch_wide(
   }
   for (u32 off = 32; off; off >>= 1) unres_total += __shfl_down(unres_total, off, 64);
   if (lane_id() == 0 && unres_total)
-    atomicAdd(reinterpret_cast<unsigned long long*>(&st->unresolved[0]), unres_total);
+    atomicAdd(reinterpret_cast<unsigned long long*>(&st->unresolved), unres_total);
 }
 
 // Large batch files after resolution: Adler-32 of each decoded file against
@@ -4645,7 +4644,7 @@ __global__ __launch_bounds__(256) void g_batch_wide_finish(const BatchFile* file
       const u32 a = u32((red[0][0] + red[0][1] + red[0][2] + red[0][3] + 1) % kAdlerMod);
       const u64 w_all = red[1][0] + red[1][1] + red[1][2] + red[1][3] + len % kAdlerMod;
       const u32 b = u32(w_all % kAdlerMod);
-      if (((b << 16) | a) == wanted[i] && !st->unresolved[1]) {
+      if (((b << 16) | a) == wanted[i]) {
         meta[2 * u64(f)] = 0;
         meta[2 * u64(f) + 1] = 0;
       } else {
@@ -4656,190 +4655,435 @@ __global__ __launch_bounds__(256) void g_batch_wide_finish(const BatchFile* file
   }
 }
 
-// Chain links a position follows in resolve round r: 2, 4, and in the last
-// round as many as its chain has (a root always precedes its position, so
-// every chain ends).  Early rounds see nearly every unresolved byte, and a
-// wave waits for its longest chain, so they take few links (measured on 64 MiB
-// of text: 2, 8, 32 took the rounds 6 % longer); each round leaves every
-// position's root as far along its chain as it got, so after two rounds a
-// chain of n links is n / 8 roots long.  Schedules of 2, 8 / 4, 16 / 4, 8, 16
-// links before the last round took as long within 3 %.
-constexpr u32 kResolveRounds = 3;
-constexpr u32 kXcds = 8;  // MI355X: 8 accelerator complex dies of 32 CUs
-__host__ __device__ constexpr u32 resolve_links(u32 round) {
-  return round == 0 ? 2u : round == 1 ? 4u : 0xffffffffu;
-}
-inline u32 resolve_rounds(u64) { return kResolveRounds; }
+// ---- resolve: stripes of the output, each by one workgroup --------------------
+// Measured on one MI355X, 64 MiB of text (47 million unresolved bytes): rounds
+// that followed every byte's roots through memory, waiting on L2 misses, took
+// 1740 us; the stripes (bound by VALU issue) 207 us, the windows 44 us and the
+// rest 134 us.  512 stripes, two workgroups per CU: 226, 196 and 139 us (a byte
+// survives a tile's walk past the stripe's start with a share that halves
+// about every 33 KiB, so short stripes leave more).
+constexpr u32 kStripeThreads = 1024;
+constexpr u32 kStripeTile = 4 * kStripeThreads;  // bytes a step resolves, four per thread
+constexpr u32 kStripeWindow = 32768;             // the longest back-reference
+constexpr u32 kStripeRing = kStripeWindow + kStripeTile;
+constexpr u32 kStripes = 256;                    // a workgroup per CU
+constexpr u64 kStripeMin = 65536;                // output bytes below which a stripe is not cut
+// A ring entry: a byte (0 .. 255), or one of
+constexpr u32 kRingPending = 0x2000u;  // | tile offset of the byte it copies, in the same tile
+constexpr u32 kRingFar = 0x4000u;      // unresolved, its chain leaves the ring and the window before
+constexpr u32 kRingBefore = 0x8000u;   // | offset in the 32 KiB before the stripe it copies from
+static_assert(kStripeTile <= 0x2000u && kStripeTile == 2u << kResolveGroupShift,
+              "tile offsets fit their tag; a tile is two mark groups");
 
-// One resolution round: round r scans the unresolved bits of buffer (r & 1)
-// (round 0: the bits set by emission; counts[r] unresolved positions,
-// zero-filled before the first round) and writes every word of the other
-// buffer with the positions still unresolved, counted in counts[r + 1].  A
-// position follows up to resolve_links(round) links of its root chain through this
-// round's snapshot (roots: any root read is an earlier byte of the same
-// chain, so concurrent updates are harmless); at a resolved byte it takes
-// that byte, else it keeps the root reached.  Round r thus covers
-// the product of resolve_links over rounds 0..r.  Only bytes written by earlier launches are
-// read.  The last round leaves its count in st->unresolved[1] (status 20 in
-// g_finish).
-// With `parts`, every resolved byte is added to this workgroup's Adler-32
-// pair parts[2b], parts[2b + 1] (a byte at position p weighs out_end - p).
-__global__ __launch_bounds__(256) void g_resolve(State* st, u8* out, u32* roots, u32* bits0,
-                                                 u32* bits1, u64* counts, u32 round,
-                                                 u32 max_rounds, u64 words, u64 out_end,
-                                                 u64* parts, u8* marks0, u8* marks1) {
-  __shared__ u64 red[2][16];
-  if (st->status || st->emit_status) return;
-  const u64 n_in = round ? counts[round] : st->unresolved[0];
-  if (!n_in) return;
-  u64 as = 0, aw = 0;
-  const u32* bits = round & 1 ? bits1 : bits0;
-  u32* next_bits = round & 1 ? bits0 : bits1;
-  u64* next_count = round + 1 == max_rounds ? &st->unresolved[1] : &counts[round + 1];
-  const u32 lane = lane_id();
-  u32 kept = 0;
-  // A wave takes a group of 64 bitmap words at a time and lists the group's
-  // unresolved positions in LDS (a prefix sum over the words' bit counts);
-  // its lanes then follow the root chains of the list's entries, 64 at a
-  // time, so that sparse and dense groups alike keep every lane busy.  The
-  // entries still unresolved are gathered into the group's next words in LDS.
-  // With group marks (marks0 for rounds 0, 2, ..., marks1 for the others), a
-  // round reads only the marked groups of its bitmap and marks those it
-  // leaves unresolved bytes in for the next round; the other groups' words
-  // of the next bitmap are never read.
-  __shared__ u16 list[256 / 64][64 * 32];
-  __shared__ u32 left_words[256 / 64][64];
-  const u32 wave = threadIdx.x >> 6;
-  const u8* marks = round & 1 ? marks1 : marks0;
-  u8* next_marks = round & 1 ? marks0 : marks1;
-  const u32 links = resolve_links(round);
-  // Workgroups are dealt to the 8 XCDs in turn (workgroup b to XCD b mod 8),
-  // each with its own L2.  XCD x takes the x-th eighth of the groups, its
-  // waves consecutive groups, so that the chains a wave follows back into
-  // the previous 32 KiB mostly read lines its own XCD's waves loaded.
-  const u64 ngroups = (words + 63) / 64;
-  // Follows the chain of entry e of group g; a byte left unresolved sets its
-  // bit in `left` (the group's next words).  The lane's stores (the byte, or
-  // the root reached) wait in `pend` until its next entry's loads have
-  // returned: a load waits for every store issued before it, so each entry's
-  // chain would otherwise wait for the previous entry's stores.
-  u32 pend_u = 0, pend_v = 0, pend_kind = 0;  // kind 1: out[u] = v; 2: roots[u] = v
-  const auto commit = [&]() {
-    if (pend_kind == 1) out[pend_u] = u8(pend_v);
-    else if (pend_kind == 2)
-      __hip_atomic_store(roots + pend_u, pend_v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    pend_kind = 0;
-  };
-  const auto chase = [&](u64 g, u32 e, u32* left) {
-    const u32 u = u32(g * 2048 + e);
-    u32 r = roots[u];
-    bool unres = (bits[r >> 5] >> (r & 31)) & 1u;
-    for (u32 k = 0; unres && k < links; ++k) {
-      r = __hip_atomic_load(roots + r, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      unres = (bits[r >> 5] >> (r & 31)) & 1u;
-    }
-    const u32 v = unres ? r : u32(out[r]);
-    commit();
-    pend_u = u;
-    pend_v = v;
-    pend_kind = unres ? 2u : 1u;
-    if (!unres) {
-      as += v;
-      aw += (out_end - u) * v;
-      if (aw >> 62) aw %= kAdlerMod;
-    } else {
-      atomicOr(&left[e >> 5], 1u << (e & 31));
-    }
-  };
-  // The group's unresolved positions into the wave's list (a prefix sum over
-  // the words' bit counts); returns their number.
-  const auto list_group = [&](u64 g, u32 m) {
-    const u32 cnt = __popc(m);
-    u32 incl = cnt;
+struct StripeShared {
+  __align__(16) u16 ring[kStripeRing];
+  u32 left[2][2];  // by tile parity: unresolved bytes remain in a mark group
+  u64 red[2][16];
+};
+
+// Four output bytes at position p (little-endian), those past `end` zero.
+__device__ __forceinline__ u32 stripe_load4(const u8* out, u64 p, u64 end, bool aligned) {
+  if (aligned && p + 4 <= end) return *reinterpret_cast<const u32*>(out + p);
+  u32 v = 0;
 #pragma unroll
-    for (u32 off = 1; off < 64; off <<= 1) {
-      const u32 y = __shfl_up(incl, off, 64);
-      if (lane >= off) incl += y;
-    }
-    for (u32 k = incl - cnt; m; m &= m - 1, ++k) list[wave][k] = u16(lane * 32 + __builtin_ctz(m));
-    return __shfl(incl, 63, 64);
+  for (u32 j = 0; j < 4; ++j)
+    if (p + j < end) v |= u32(out[p + j]) << (8 * j);
+  return v;
+}
+
+// Adds a workgroup's Adler-32 pairs to the slots of `parts`.
+__device__ __forceinline__ void resolve_add_parts(u64* parts, u64 as, u64 aw, u64 (*red)[16]) {
+  adler_block_sum(as, aw, red);
+  if (!threadIdx.x && (as | aw)) {
+    const u32 slot = blockIdx.x % kAdlerSlots;
+    atomicAdd(reinterpret_cast<unsigned long long*>(&parts[2 * slot]), as);
+    atomicAdd(reinterpret_cast<unsigned long long*>(&parts[2 * slot + 1]), aw);
+  }
+}
+
+// Four output bytes of a stripe's thread with their unresolved bits and roots,
+// loaded a tile ahead: straight-line loads, nothing computed from them here,
+// so that no wait stands between them and the tile being worked on.
+struct StripeLoad {
+  u32 word, w0, w1;
+  uint4 roots;
+  // words: the output's aligned dwords, of which dword `last` is the last one.
+  __device__ __forceinline__ void load(const u32* words, u32 skew, u32 last, const u32* root,
+                                       const u32* bits, u32 p) {
+    const u32 q = (p + skew) >> 2;  // p is a multiple of 4
+    word = bits[p >> 5];
+    w0 = words[q];
+    w1 = words[min(q + 1, last)];
+    roots = *reinterpret_cast<const uint4*>(root + p);
+  }
+};
+
+// Below one unresolved byte in this many the stripes are skipped: the chains
+// are few, and following them one by one (g_resolve_windows, g_resolve_rest)
+// costs less than walking the tiles (the 64 MiB strain stream: 57 us
+// against 162).
+constexpr u64 kStripeSparse = 64;
+
+// Resolves most unresolved bytes: workgroup b walks stripe b of the output in
+// 4 KiB tiles, in order, with the marked tiles of the last 32 KiB of the
+// stripe in an LDS ring.  A tile's unresolved bytes take their root's value
+// from the ring (from the output, where the root's tile had no mark) or by
+// pointer jumping over roots inside the tile, all in LDS; a root before the
+// stripe stays one, tagged in the ring, and passes through every copy of it.
+// Only bytes whose chain ends before the stripe stay unresolved, with that end
+// as their root, and those whose chain meets a root more than 32 KiB back (a
+// run's), which keep the root they had.  The barriers of a tile order LDS only, so that the next tile's
+// loads stay in flight over them.
+// Bits, marks and roots are updated in place; the bytes left are counted in
+// *left_count.  With `parts`, every byte resolved is added to the Adler-32
+// pairs (a byte at position p weighs out_end - p).
+__global__ __launch_bounds__(kStripeThreads) __attribute__((amdgpu_waves_per_eu(8))) void
+g_resolve_stripes(State* st, u8* out, u32* roots, u32* bits, u8* marks, u64 out_end,
+                  u64 stripe_bytes, u64* left_count, u64* parts) {
+  __shared__ StripeShared sh;
+  if (st->status || st->emit_status) return;
+  const u32 t = threadIdx.x, lane = lane_id();
+  if (gridDim.x > 1 && st->unresolved < out_end / kStripeSparse) {
+    if (!blockIdx.x && !t) *left_count = st->unresolved;
+    return;
+  }
+  if (!st->unresolved) return;
+  constexpr u32 kRingTiles = kStripeRing / kStripeTile;
+  const u64 start = u64(blockIdx.x) * stripe_bytes;
+  const u64 end = min(start + stripe_bytes, out_end);
+  const u32 tiles = u32((end - start + kStripeTile - 1) / kStripeTile);
+  const u32 skew = u32(reinterpret_cast<uintptr_t>(out) & 3u);
+  const u32* words = reinterpret_cast<const u32*>(out - skew);
+  const u32 last = u32((out_end - 1 + skew) >> 2);
+  const u32 groups = u32((out_end + (1u << kResolveGroupShift) - 1) >> kResolveGroupShift);
+  u8* bit_bytes = reinterpret_cast<u8*>(bits);
+  if (t < 4) sh.left[t >> 1][t & 1] = 0;
+  __syncthreads();
+  // Marked tiles, 32 tiles of marks (two each) at a time, the same in every
+  // wave.
+  u32 tb = 0;
+  u64 marked = 0;
+  const auto load_marks = [&]() {
+    const u32 mg = u32(start >> kResolveGroupShift) + 2 * tb + lane;
+    marked = __ballot(mg < groups && 2 * tb + lane < 2 * tiles && marks[mg]);
   };
-  if (ngroups <= gridDim.x) {  // uniform
-    // Few groups (a small output): a workgroup per group, its four waves
-    // chasing every fourth batch of 64 entries, so that a group's chains are
-    // followed four times as fast.  Each wave lists the group itself.
-    for (u64 g = blockIdx.x; g < ngroups; g += gridDim.x) {
-      if (marks && !marks[g]) {  // uniform
-        if (!threadIdx.x) next_marks[g] = 0;
-        continue;
-      }
-      const u64 w = g * 64 + lane;
-      const u32 total = list_group(g, w < words ? bits[w] : 0u);
-      if (!total) {  // uniform
-        if (!wave && w < words) next_bits[w] = 0;
-        if (marks && !threadIdx.x) next_marks[g] = 0;
-        continue;
-      }
-      if (!wave) left_words[0][lane] = 0;
-      __syncthreads();
-      for (u32 i = wave * 64 + lane; i < total; i += 256) chase(g, list[wave][i], left_words[0]);
-      commit();
-      __syncthreads();
-      if (!wave) {
-        const u32 nb = left_words[0][lane];
-        if (w < words) next_bits[w] = nb;
-        kept += __popc(nb);
-        const bool left = __ballot(nb != 0) != 0;
-        if (marks && !lane) next_marks[g] = left ? 1 : 0;
-      }
-      __syncthreads();  // the list and words are rewritten for the next group
+  const auto next_tile = [&]() -> u32 {
+    while (!marked) {
+      tb += 32;
+      if (tb >= tiles) return kNone;
+      load_marks();
     }
-  } else {
-    // Workgroups are dealt to the 8 XCDs in turn (workgroup b to XCD b mod
-    // 8), each with its own L2.  XCD x takes the x-th eighth of the groups,
-    // its waves consecutive groups, so that the chains a wave follows back
-    // into the previous 32 KiB mostly read lines its own XCD's waves loaded.
-    const u32 xcds = gridDim.x < kXcds ? gridDim.x : kXcds;
-    const u32 xcd = blockIdx.x % xcds, xcd_block = blockIdx.x / xcds;
-    const u64 xcd_waves =
-        u64(gridDim.x / xcds + (xcd < gridDim.x % xcds ? 1u : 0u)) * (blockDim.x / 64);
-    const u64 g_end = ngroups * (xcd + 1) / xcds;
-    for (u64 g = ngroups * xcd / xcds + u64(xcd_block) * (blockDim.x / 64) + wave; g < g_end;
-         g += xcd_waves) {
-      if (marks && !marks[g]) {  // uniform
-        if (!lane) next_marks[g] = 0;
-        continue;
-      }
-      const u64 w = g * 64 + lane;
-      const u32 total = list_group(g, w < words ? bits[w] : 0u);
-      if (!total) {  // uniform
-        if (w < words) next_bits[w] = 0;
-        if (marks && !lane) next_marks[g] = 0;
-        continue;
-      }
-      left_words[wave][lane] = 0;
-      wave_sync();
-      for (u32 i = lane; i < total; i += 64) chase(g, list[wave][i], left_words[wave]);
-      commit();
-      wave_sync();
-      const u32 nb = left_words[wave][lane];
-      if (w < words) next_bits[w] = nb;
-      kept += __popc(nb);
-      const bool left = __ballot(nb != 0) != 0;
-      if (marks && !lane) next_marks[g] = left ? 1 : 0;
-      wave_sync();  // the list and words are rewritten for the next group
+    const u32 b = u32(__builtin_ctzll(marked)) / 2;
+    marked &= ~(3ull << (2 * b));
+    return tb + b;
+  };
+  const auto load_tile = [&](StripeLoad& l, u32 tile) {  // any tile of the stripe
+    const u32 p = u32(start) + tile * kStripeTile + 4 * t;
+    l.load(words, skew, last, roots, bits, min(p, u32(end - 1) & ~3u));
+  };
+  load_marks();
+  u32 ti = next_tile();
+  u32 have = 0, parity = 0, kept = 0;  // have: bit k: tile ti - 1 - k is in the ring
+  u64 as = 0, aw = 0;
+  StripeLoad cur, nxt;
+  if (ti != kNone) load_tile(cur, ti);
+  while (ti != kNone) {  // uniform
+    const u32 ti2 = next_tile();
+    load_tile(nxt, ti2 != kNone ? ti2 : ti);
+    // Positions in 32 bits, as the roots are.
+    const u32 start32 = u32(start), tile0 = start32 + ti * kStripeTile, p = tile0 + 4 * t;
+    const u32 slot0 = (ti % kRingTiles) * kStripeTile;
+    u32 nib = p < u32(end) ? (cur.word >> (p & 31u)) & 15u : 0u;
+    const u32 bytes = __builtin_amdgcn_alignbyte(cur.w1, cur.w0, skew);
+    u32 e[4], r[4] = {cur.roots.x, cur.roots.y, cur.roots.z, cur.roots.w};
+    u32 direct = 0;  // bytes whose root's tile is not in the ring
+#pragma unroll
+    for (u32 j = 0; j < 4; ++j) {
+      const u32 x = r[j], d = tile0 - x;  // bytes from the root to the tile (wraps inside it)
+      const bool unres = (nib >> j) & 1u, inside = x >= start32, tile = x >= tile0;
+      const bool near = inside && !tile && d <= kStripeWindow;
+      const u32 slot = near ? slot0 - d + (slot0 >= d ? 0u : kStripeRing) : 0u;
+      const u32 ring = sh.ring[slot];
+      const u32 other = tile ? kRingPending | (x - tile0)
+                        : !inside && start32 - x <= kStripeWindow
+                            ? kRingBefore | (x + kStripeWindow - start32) : kRingFar;
+      e[j] = unres ? (near ? ring : other) : (bytes >> (8 * j)) & 255u;
+      const bool held = (have >> (((d - 1) / kStripeTile) & 31u)) & 1u;
+      direct |= u32(unres && near && !held) << j;
     }
+    if (direct) {
+      u32 v[4];
+#pragma unroll
+      for (u32 j = 0; j < 4; ++j) v[j] = out[(direct >> j) & 1u ? r[j] : tile0];
+#pragma unroll
+      for (u32 j = 0; j < 4; ++j) {
+        e[j] = (direct >> j) & 1u ? v[j] : e[j];
+        asm volatile("" : "+v"(e[j]));  // these loads are waited for here, not past the branch
+      }
+    }
+    // Chains inside the tile by pointer jumping: every link is an earlier
+    // byte; entries are rewritten as they advance or end, and a chain read
+    // while others advance only gets shorter.
+    const auto store = [&]() {
+      *reinterpret_cast<uint2*>(&sh.ring[slot0 + 4 * t]) =
+          make_uint2(e[0] | (e[1] << 16), e[2] | (e[3] << 16));
+    };
+    store();
+    lds_barrier();
+    for (;;) {
+      u32 at[4];
+      bool more = false;
+#pragma unroll
+      for (u32 j = 0; j < 4; ++j) {
+        const bool pending = e[j] - kRingPending < kStripeTile;
+        at[j] = slot0 + (pending ? e[j] - kRingPending : 4 * t + j);  // an ended one reads itself
+        more |= pending;
+      }
+      if (!__ballot(more)) break;
+#pragma unroll
+      for (u32 j = 0; j < 4; ++j)
+        e[j] = __hip_atomic_load(&sh.ring[at[j]], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      store();
+    }
+    if (nib) {
+      u32 rem = 0, v = 0, cs = 0, cl = 0;
+#pragma unroll
+      for (u32 j = 0; j < 4; ++j) {
+        if (e[j] & kRingBefore) r[j] = start32 - kStripeWindow + (e[j] & (kRingBefore - 1u));
+        if (e[j] >= kRingFar) rem |= 1u << j;
+        else v |= e[j] << (8 * j);
+        const u32 x = ((nib & ~rem) >> j) & 1u ? e[j] : 0u;
+        cs += x;
+        cl += j * x;
+      }
+      as += cs;
+      aw += (out_end - p) * cs - cl;
+      if (aw >> 60) aw %= kAdlerMod;
+      if (!skew && p + 4 <= u32(end)) {
+        *reinterpret_cast<u32*>(out + p) = v;
+      } else {
+#pragma unroll
+        for (u32 j = 0; j < 4; ++j)
+          if ((nib >> j) & 1u) out[p + j] = u8(v >> (8 * j));
+      }
+      if (rem) {
+        // Bytes that are resolved have no root: the whole line is this thread's.
+        *reinterpret_cast<uint4*>(roots + p) = make_uint4(r[0], r[1], r[2], r[3]);
+        sh.left[parity][t / (kStripeThreads / 2)] = 1;
+        kept += __popc(rem);
+      }
+      nib = rem | 0x10u;  // changed
+    }
+    // Two threads' bits make a byte of the bitmap.
+    const u32 other = __shfl_xor(nib, 1, 64);
+    if (!(t & 1u) && ((nib | other) & 0x10u)) bit_bytes[p >> 3] = u8((nib & 15u) | (other << 4));
+    lds_barrier();
+    if (t < 2) {
+      const u32 g = (tile0 >> kResolveGroupShift) + t;
+      if (g < groups) marks[g] = u8(sh.left[parity][t]);
+      sh.left[parity][t] = 0;  // next set two tiles on
+    }
+    parity ^= 1;
+    const u32 step = ti2 - ti;  // tiles without a mark are not in the ring
+    have = step < 32 ? ((have << 1 | 1u) << (step - 1)) & ((1u << (kRingTiles - 1)) - 1u) : 0u;
+    ti = ti2;
+    cur = nxt;
+  }
+  if (gridDim.x == 1 && __syncthreads_or(kept)) {
+    // The only stripe: far bytes, followed to a resolved one (no bit changes
+    // any more, and every store before is visible past the barrier).
+    for (u64 p = 8 * u64(t); p < end; p += 8 * kStripeThreads)
+      for (u32 m = bit_bytes[p >> 3]; m; m &= m - 1) {
+        const u64 u = p + u32(__builtin_ctz(m));
+        u32 x = roots[u];
+        while ((bit_bytes[x >> 3] >> (x & 7)) & 1u) x = roots[x];
+        const u32 v = out[x];
+        out[u] = u8(v);
+        as += v;
+        aw += (out_end - u) * v;
+        if (aw >> 60) aw %= kAdlerMod;
+      }
   }
   for (u32 off = 32; off; off >>= 1) kept += __shfl_down(kept, off, 64);
-  if (lane_id() == 0 && kept) atomicAdd(reinterpret_cast<unsigned long long*>(next_count), u64(kept));
-  if (parts) {  // uniform
-    adler_block_sum(as, aw, red);
-    if (!threadIdx.x) {
-      const u32 slot = blockIdx.x % kAdlerSlots;
-      atomicAdd(reinterpret_cast<unsigned long long*>(&parts[2 * slot]), as);
-      atomicAdd(reinterpret_cast<unsigned long long*>(&parts[2 * slot + 1]), aw);
+  if (!lane && kept) atomicAdd(reinterpret_cast<unsigned long long*>(left_count), u64(kept));
+  if (parts) resolve_add_parts(parts, as, aw, sh.red);
+}
+
+// The bytes g_resolve_stripes left in the last 32 KiB of every stripe but the
+// last: the windows that nearly all other bytes left are rooted in.  One
+// workgroup per mark group, eight chains a thread side by side (a wave's 64
+// positions are consecutive).  Bits stay as the stripes left them, so a chain
+// ends at the first byte the stripes had resolved.  A chain has about one link
+// per stripe it crosses; of text hardly any has two.  With `shorten`, run
+// before when most bytes were left (data that repeats itself over many
+// stripes), only the roots move, up to kShortenLinks links along their chains
+// (a root read while it moves is another byte of the same chain).
+constexpr u32 kShortenLinks = 8;
+constexpr u32 kWindowGroups = kStripeWindow >> kResolveGroupShift;
+__global__ __launch_bounds__(256) void g_resolve_windows(const State* st, u8* out, u32* roots,
+                                                         const u32* bits, const u8* marks,
+                                                         u64 out_end, u64 stripe_bytes,
+                                                         const u64* left_count, u32 shorten,
+                                                         u64* parts) {
+  __shared__ u64 red[2][16];
+  if (st->status || st->emit_status || !*left_count) return;
+  if (shorten && *left_count < out_end / 2) return;
+  const u64 g = ((blockIdx.x / kWindowGroups + 1) * stripe_bytes >> kResolveGroupShift) -
+                kWindowGroups + blockIdx.x % kWindowGroups;
+  if (!marks[g]) return;  // uniform; the group lies before the last stripe
+  constexpr u32 kPer = (1u << kResolveGroupShift) / 256;
+  const u32 p = u32(g << kResolveGroupShift) + threadIdx.x;
+  u32 r[kPer], mine = 0;
+#pragma unroll
+  for (u32 k = 0; k < kPer; ++k) {
+    const u32 u = p + 256 * k;
+    const bool unres = (bits[u >> 5] >> (u & 31)) & 1u;
+    r[k] = unres ? roots[u] : 0u;
+    mine |= u32(unres) << k;
+  }
+  u32 open = mine;  // chains not at their end
+  for (u32 link = 0; open && !(shorten && link == kShortenLinks); ++link) {
+    // A link's bit and the root past it load together (of a resolved byte the
+    // root is not used).
+    u32 b[kPer], n[kPer];
+#pragma unroll
+    for (u32 k = 0; k < kPer; ++k) {
+      if (!((open >> k) & 1u)) continue;
+      b[k] = bits[r[k] >> 5];
+      n[k] = __hip_atomic_load(roots + r[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+#pragma unroll
+    for (u32 k = 0; k < kPer; ++k) {
+      if (!((open >> k) & 1u)) continue;
+      if ((b[k] >> (r[k] & 31)) & 1u) r[k] = n[k];
+      else open &= ~(1u << k);
     }
   }
+  u64 as = 0, aw = 0;
+#pragma unroll
+  for (u32 k = 0; k < kPer; ++k) {
+    if (!((mine >> k) & 1u)) continue;
+    const u32 u = p + 256 * k;
+    if (shorten) {
+      __hip_atomic_store(roots + u, r[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    } else {
+      const u32 v = out[r[k]];
+      out[u] = u8(v);
+      as += v;
+      aw += (out_end - u) * v;
+    }
+  }
+  if (parts && !shorten) resolve_add_parts(parts, as, aw, red);
+}
+
+// The end of a root's chain once the windows are done: a byte of some
+// stripe's window, or one the stripes resolved.
+__device__ __forceinline__ u32 rest_end(const u32* bits, const u32* roots, u32 x, u64 stripe_bytes,
+                                        u64 out_end) {
+  while ((bits[x >> 5] >> (x & 31)) & 1u) {
+    const u64 in = x % stripe_bytes;
+    if (in + kStripeWindow >= stripe_bytes && x - in + stripe_bytes < out_end) break;
+    x = roots[x];
+  }
+  return x;
+}
+
+// The other bytes g_resolve_stripes left: their roots lie in the 32 KiB before
+// their stripe (final by now), or elsewhere (a run's, or with the stripes
+// skipped) and are followed.  A workgroup sweeps kRestBytes of a stripe: with
+// few bytes left there it lists them and takes one a thread, else four
+// consecutive positions a thread.
+constexpr u32 kXcds = 8;  // MI355X: 8 accelerator complex dies of 32 CUs
+constexpr u32 kRestThreads = 512;
+constexpr u32 kRestBytes = 16384;
+constexpr u32 kRestList = 4 * kRestThreads;
+static_assert(4 * kRestThreads == 1u << kResolveGroupShift, "a step is a mark group");
+__global__ __launch_bounds__(kRestThreads) void g_resolve_rest(const State* st, u8* out,
+                                                               const u32* roots, const u32* bits,
+                                                               const u8* marks, u64 out_end,
+                                                               u64 stripe_bytes, u32 parts_per,
+                                                               const u64* left_count, u64* parts) {
+  __shared__ u64 red[2][16];
+  __shared__ u16 list[kRestList];
+  __shared__ u32 listed;
+  if (st->status || st->emit_status || !*left_count) return;
+  const u32 t = threadIdx.x, lane = lane_id();
+  // Workgroups go to the 8 XCDs in turn: a stripe's stay on one, whose L2
+  // then holds the window they read.
+  const u32 slot = blockIdx.x / kXcds;
+  const u64 start = u64(slot / parts_per * kXcds + blockIdx.x % kXcds) * stripe_bytes;
+  if (start >= out_end) return;  // uniform
+  const u64 lo = start + u64(slot % parts_per) * kRestBytes;
+  // The stripe's own window is done, except the last stripe's.
+  u64 hi = min(start + stripe_bytes, out_end);
+  if (start + stripe_bytes < out_end) hi -= kStripeWindow;
+  hi = min<u64>(hi, lo + kRestBytes);
+  if (lo >= hi) return;  // uniform
+  const u64 g0 = lo >> kResolveGroupShift;
+  const u32 ng = u32((hi - lo + (1u << kResolveGroupShift) - 1) >> kResolveGroupShift);  // <= 16
+  const u32 marked = u32(__ballot(lane < ng && marks[g0 + lane]));
+  if (!marked) return;  // uniform
+  if (!t) listed = 0;
+  __syncthreads();
+  u64 as = 0, aw = 0;
+  // Two bitmap words a thread (hi is a multiple of 4096 or the output's end,
+  // whose bitmap has a word more).
+  const u32 w = 2 * t;
+  const bool has = lo + 32 * w < hi && (marked >> (w / 64)) & 1u;
+  const u64* pair = reinterpret_cast<const u64*>(bits + (lo >> 5)) + t;
+  u64 m = has ? *pair : 0;
+  const u32 n = __popcll(m);
+  u32 at = n ? atomicAdd(&listed, n) : 0;
+  for (; m && at < kRestList; m &= m - 1) list[at++] = u16(32 * w + u32(__builtin_ctzll(m)));
+  __syncthreads();
+  const u32 total = listed;
+  if (total <= kRestList) {  // uniform
+    for (u32 i = t; i < total; i += kRestThreads) {
+      const u32 u = u32(lo) + list[i];
+      const u32 v = out[rest_end(bits, roots, roots[u], stripe_bytes, out_end)];
+      out[u] = u8(v);
+      as += v;
+      aw += (out_end - u) * v;
+    }
+  } else {
+    const bool aligned = (reinterpret_cast<uintptr_t>(out) & 3u) == 0;
+    const u64 w0 = start - kStripeWindow;  // wraps for stripe 0: every root is followed
+    for (u64 p = lo + 4 * t; p < hi; p += 4 * kRestThreads) {  // a mark group a step
+      if (!((marked >> ((p - lo) >> kResolveGroupShift)) & 1u)) continue;
+      const u32 nib = (bits[p >> 5] >> (p & 31u)) & 15u;
+      if (!nib) continue;
+      const uint4 rv = *reinterpret_cast<const uint4*>(roots + p);
+      const u32 r[4] = {rv.x, rv.y, rv.z, rv.w};
+      u32 v = nib == 15u ? 0u : stripe_load4(out, p, out_end, aligned);
+      u32 x[4], b[4], cs = 0, cl = 0;
+#pragma unroll
+      for (u32 j = 0; j < 4; ++j) {
+        x[j] = 0;
+        if (!((nib >> j) & 1u)) continue;
+        x[j] = r[j] >= w0 && r[j] < start ? r[j]
+                                          : rest_end(bits, roots, r[j], stripe_bytes, out_end);
+      }
+#pragma unroll
+      for (u32 j = 0; j < 4; ++j) b[j] = out[x[j]];
+#pragma unroll
+      for (u32 j = 0; j < 4; ++j) {
+        if (!((nib >> j) & 1u)) continue;
+        v = (v & ~(255u << (8 * j))) | (b[j] << (8 * j));
+        cs += b[j];
+        cl += j * b[j];
+      }
+      as += cs;
+      aw += (out_end - p) * cs - cl;
+      if (aligned && p + 4 <= hi) {
+        *reinterpret_cast<u32*>(out + p) = v;
+      } else {
+#pragma unroll
+        for (u32 j = 0; j < 4; ++j)
+          if ((nib >> j) & 1u) out[p + j] = u8(v >> (8 * j));
+      }
+    }
+  }
+  if (parts) resolve_add_parts(parts, as, aw, red);
 }
 
 constexpr u32 kCrcTile = 16384;  // output bytes per CRC-32 tile (256 threads x 64)
@@ -4931,7 +5175,7 @@ __device__ u32 crc_from_tiles(const u64* parts, u64 n) {
 // decode, or unresolved references) is read by every workgroup: on a decode
 // error each zeroes its grid-stride share of out[0..n).  Workgroup 0 then
 // checks the trailer (`check`): Adler-32 from the `nparts` pairs the emitters
-// and resolve rounds accumulated (every output byte is summed once, by
+// and resolve kernels accumulated (every output byte is summed once, by
 // whichever kernel wrote it), CRC-32 and size from g_crc_tiles' tile
 // registers, or nothing, and writes the metadata.  A trailer mismatch keeps
 // the output.
@@ -4947,8 +5191,6 @@ __global__ __launch_bounds__(256) void g_finish(State* st, u64 n, u32* meta, con
   const u32 t = threadIdx.x, lane = lane_id(), wave = t >> 6;
   u32 status = st->status;
   if (!status) status = st->emit_status;
-  // References still unresolved after every round.
-  if (!status && st->unresolved[1]) status = kReferenceDepth;
   if (status && !open.open) {  // uniform; st->status never holds a trailer mismatch here
     const u64 stride = u64(gridDim.x) * blockDim.x;
     for (u64 i = u64(blockIdx.x) * blockDim.x + t; i < n; i += stride) out[i] = 0;
@@ -5018,6 +5260,33 @@ u32 clamp_grid(u64 want, u32 cap) { return u32(want < 1 ? 1 : (want > cap ? cap 
   } while (0)
 }  // namespace
 
+namespace {
+// Resolution of the unresolved bytes of out[0, total): the stripes, then the
+// bytes they leave, first those in the stripes' windows.  With one stripe
+// nothing is left.  left: a zeroed counter.
+hipError_t launch_resolve(hipStream_t stream, State* st, u8* out, u32* roots, u32* bits, u8* marks,
+                          u64* left, u64 total, u64* parts) {
+  if (!total) return hipSuccess;
+  const u64 want = std::min<u64>(kStripes, (total + kStripeMin - 1) / kStripeMin);
+  const u64 stripe = ((total + want - 1) / want + kStripeTile - 1) / kStripeTile * kStripeTile;
+  const u32 stripes = u32((total + stripe - 1) / stripe);
+  HZ_LAUNCH(g_resolve_stripes, dim3(stripes), dim3(kStripeThreads), 0, stream, st, out, roots, bits,
+            marks, total, stripe, left, parts);
+  HZ_TRY(hipGetLastError());
+  if (stripes == 1) return hipSuccess;
+  for (u32 shorten = stripes > kShortenLinks ? 1 : 0;; shorten = 0) {
+    HZ_LAUNCH(g_resolve_windows, dim3((stripes - 1) * kWindowGroups), dim3(256), 0, stream, st, out,
+              roots, bits, marks, total, stripe, left, shorten, parts);
+    HZ_TRY(hipGetLastError());
+    if (!shorten) break;
+  }
+  const u32 per = u32((stripe + kRestBytes - 1) / kRestBytes);
+  HZ_LAUNCH(g_resolve_rest, dim3((stripes + kXcds - 1) / kXcds * kXcds * per), dim3(kRestThreads),
+            0, stream, st, out, roots, bits, marks, total, stripe, per, left, parts);
+  return hipGetLastError();
+}
+}  // namespace
+
 hipError_t run_inflate_general(hipStream_t stream, Scratch& scratch, const u8* in, u64 in_size,
                                u8* out, u64 out_size, u32 max_candidates, u32 max_blocks,
                                u32* meta, const StreamFormat& fmt) {
@@ -5037,21 +5306,18 @@ hipError_t run_inflate_general(hipStream_t stream, Scratch& scratch, const u8* i
   u8* stream_out = out + out_base;
   State* st = nullptr;
   HZ_TRY(scratch.alloc(&st, 1));
-  // Emission and resolution scratch sizes.  A resolve chain hops back across
-  // slices (or serially emitted segments), so its length is bounded by the
-  // number of slices plus segments.
+  // Emission and resolution scratch sizes.
   const u64 group_capacity = (len * 8) / 8192 + 65536;
   const u64 words = (out_total + 31) / 32 + 1;
-  const u32 rounds = resolve_rounds(group_capacity * 64 + u64(max_blocks));
   // Fixed-run tiles of the body and their bitmap (zeroed with the rest).
   const u64 tiles = (len * 8 + kFixTileBits - 1) / kFixTileBits;
   const u64 need_words = tiles / 32 + 1;
   // Adler-32 partial pairs: kAdlerSlots each for the lane emitter, the
-  // serial emitter and the resolve rounds (workgroups add theirs, so they
-  // start at zero), summed by g_finish.  The pairs, the round counts and the
-  // first unresolved bitmap are zeroed by g_frame.
+  // serial emitter and the resolve kernels (workgroups add theirs, so they
+  // start at zero), summed by g_finish.  The pairs, the count of bytes left and the
+  // unresolved bitmap are zeroed by g_frame.
   u8* zeroed = nullptr;
-  const u64 zero_u64 = 2 * u64(3 * kAdlerSlots) + rounds + 1;
+  const u64 zero_u64 = 2 * u64(3 * kAdlerSlots) + 1;
   // Resolve group marks (emission marks groups in marks0).
   const u64 mark_groups_n = (words + 63) / 64;
   const u64 zero_bytes = 8 * zero_u64 + 4 * words + 4 * need_words + (mark_groups_n + 3) / 4 * 4;
@@ -5202,18 +5468,12 @@ hipError_t run_inflate_general(hipStream_t stream, Scratch& scratch, const u8* i
 
   // Emission and cross-segment resolution.
   const u32 emit_grid = clamp_grid(std::min<u64>(max_blocks, items_cap), 4096);
-  // A workgroup per group of 64 words while there are at most 2048 groups
-  // (g_resolve then shares each group among its waves), else 2048.
-  const u32 resolve_grid = clamp_grid((words + 63) / 64, 2048);
   u64* adler_parts = reinterpret_cast<u64*>(zeroed);
-  u64* counts = adler_parts + 2 * u64(3 * kAdlerSlots);
-  u32* bits0 = reinterpret_cast<u32*>(counts + rounds + 1);
-  u32 *roots = nullptr, *bits1 = nullptr;
+  u64* left = adler_parts + 2 * u64(3 * kAdlerSlots);
+  u32* bits0 = reinterpret_cast<u32*>(left + 1);
+  u32* roots = nullptr;
   HZ_TRY(scratch.alloc(&roots, out_total ? out_total : 1));
-  HZ_TRY(scratch.alloc(&bits1, words));
   u8* marks0 = zeroed + 8 * zero_u64 + 4 * words + 4 * need_words;
-  u8* marks1 = nullptr;
-  HZ_TRY(scratch.alloc(&marks1, mark_groups_n));
   const u64 out_end = out_total;  // a byte at position p is stream byte n - (out_end - p)
   // Emission by segments, then the queued units of long fixed runs.
   EmitUnit* units = nullptr;
@@ -5228,16 +5488,13 @@ hipError_t run_inflate_general(hipStream_t stream, Scratch& scratch, const u8* i
   HZ_LAUNCH(g_emit_serial, dim3(emit_grid), dim3(kWave), 0, stream, body, len, st, acc, out,
             roots, bits0, out_end, adler_parts + 2 * kAdlerSlots, marks0);
   HZ_TRY(hipGetLastError());
-  for (u32 round = 0; round < rounds; ++round) {
-    HZ_LAUNCH(g_resolve, dim3(resolve_grid), dim3(256), 0, stream, st, out, roots, bits0, bits1,
-              counts, round, rounds, words, out_end, adler_parts + 4 * kAdlerSlots, marks0, marks1);
-    HZ_TRY(hipGetLastError());
-  }
+  HZ_TRY(launch_resolve(stream, st, out, roots, bits0, marks0, left, out_end,
+                        adler_parts + 4 * kAdlerSlots));
   u64* parts = nullptr;
   u32 nparts = 0;
   const u32 finish_grid = clamp_grid((out_size + 255) / 256, 4096);
   if (check == kCheckAdler) {
-    // The pairs of the emitters, then those of the resolve rounds.
+    // The pairs of the emitters, then those of the resolve kernels.
     HZ_LAUNCH(g_finish, dim3(finish_grid), dim3(256), 0, stream, st, out_size, meta, adler_parts,
               3 * kAdlerSlots, check, stream_out, open, body, body_off, fmt.report);
     return hipGetLastError();
@@ -5266,37 +5523,33 @@ hipError_t run_inflate_batch_wide(hipStream_t stream, Scratch& scratch, const u8
   // the partly filled last group of every describe round.
   const u64 group_capacity = in_bits / (u64(kDescMinSlice) * 64) +
                              in_bits / (u64(kDescThreads) * kDescMinSlice) + 8 * u64(n) + 64;
-  const u32 rounds = resolve_rounds(group_capacity * 64 + u64(max_blocks));
   const u64 words = (out_total + 31) / 32 + 1;
-  // The state, the resolve counts and the first bitmap start zeroed: one
-  // allocation, cleared by one fill.
+  const u64 mark_groups_n = (words + 63) / 64;
+  // The state, the count of bytes the stripes leave, the bitmap and its group marks start
+  // zeroed: one allocation, cleared by one fill.
   const u64 st_bytes = scratch_round(sizeof(State));
-  const u64 counts_bytes = scratch_round((rounds + 1) * sizeof(u64));
+  const u64 left_bytes = scratch_round(sizeof(u64));
+  const u64 zero_bytes = st_bytes + left_bytes + words * 4 + mark_groups_n;
   u8* zeroed = nullptr;
-  HZ_TRY(scratch.alloc(&zeroed, st_bytes + counts_bytes + words * 4));
-  HZ_TRY(launch_fill(stream, zeroed, 0, st_bytes + counts_bytes + words * 4));
+  HZ_TRY(scratch.alloc(&zeroed, zero_bytes));
+  HZ_TRY(launch_fill(stream, zeroed, 0, zero_bytes));
   State* st = reinterpret_cast<State*>(zeroed);
-  u64* counts = reinterpret_cast<u64*>(zeroed + st_bytes);
-  u32* bits0 = reinterpret_cast<u32*>(zeroed + st_bytes + counts_bytes);
+  u64* left = reinterpret_cast<u64*>(zeroed + st_bytes);
+  u32* bits0 = reinterpret_cast<u32*>(zeroed + st_bytes + left_bytes);
+  u8* marks0 = zeroed + st_bytes + left_bytes + words * 4;
   u64* slice_entry = nullptr;
   u32 *slice_off = nullptr, *group_link = nullptr, *wanted = nullptr;
   HZ_TRY(scratch.alloc(&slice_entry, group_capacity * 64));
   HZ_TRY(scratch.alloc(&slice_off, group_capacity * 64));
   HZ_TRY(scratch.alloc(&group_link, group_capacity));
   HZ_TRY(scratch.alloc(&wanted, u64(n) + 1));
-  u32 *roots = nullptr, *bits1 = nullptr;
+  u32* roots = nullptr;
   HZ_TRY(scratch.alloc(&roots, out_total ? out_total : 1));
-  HZ_TRY(scratch.alloc(&bits1, words));
   HZ_LAUNCH(g_batch_wide, dim3(n), dim3(kDescThreads), 0, stream, in, out, files, list, n,
             encoded, max_blocks, st, slice_entry, slice_off, group_link, group_capacity, roots,
-            bits0, redo, wanted);
+            bits0, redo, wanted, marks0);
   HZ_TRY(hipGetLastError());
-  for (u32 round = 0; round < rounds; ++round) {
-    HZ_LAUNCH(g_resolve, dim3(u32(clamp_grid((words + 255) / 256, 2048))), dim3(256), 0, stream,
-              st, out, roots, bits0, bits1, counts, round, rounds, words, 0ull, nullptr, nullptr,
-              nullptr);
-    HZ_TRY(hipGetLastError());
-  }
+  HZ_TRY(launch_resolve(stream, st, out, roots, bits0, marks0, left, out_total, nullptr));
   HZ_LAUNCH(g_batch_wide_finish, dim3(n), dim3(256), 0, stream, files, list, n, out, st, wanted,
             redo, meta);
   return hipGetLastError();

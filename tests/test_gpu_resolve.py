@@ -1,0 +1,86 @@
+"""Back-reference resolution by output stripes: sizes around the tile, window and
+stripe edges, with chains inside a tile, across tiles and across stripes."""
+
+import zlib
+
+import numpy as np
+import pytest
+
+import workloads
+
+pytestmark = pytest.mark.gpu
+
+TILE, STRIPE = 4096, 65536
+
+
+def _content(kind, n):
+    rng = np.random.default_rng(n)
+    if kind == "text":
+        return workloads.text_like(n, rng)
+    if kind == "period":  # every byte copies from one period back, over all stripes
+        block = rng.integers(0, 256, 32000, dtype=np.uint8).tobytes()
+        return (block * (n // len(block) + 1))[:n]
+    if kind == "runs":  # run bytes rooted further back than the window
+        return workloads.runs_segment(n, rng)
+    # Mostly literals with a few copies (below the density the stripes are walked at).
+    data = rng.integers(0, 256, n, dtype=np.uint8)
+    for _ in range(n // 2000):
+        at = int(rng.integers(100, n - 40))
+        back = int(rng.integers(1, min(at, 30000) + 1))
+        data[at:at + 40] = np.resize(data[at - back:at], 40)
+    return data.tobytes()
+
+
+@pytest.mark.parametrize("kind", ["text", "period", "runs", "sparse"])
+@pytest.mark.parametrize("size", [TILE - 1, TILE + 1, 32768 + TILE + 3, STRIPE, STRIPE + 1,
+                                  2 * STRIPE + TILE + 2, 20 * STRIPE + 4093])
+def test_resolved_output(gpu, kind, size):
+    import cuda_zlib
+    raw = _content(kind, size)
+    payload = zlib.compress(raw, 6)
+    out, meta = cuda_zlib.decompress_zlib_checked(payload, len(raw), gpu)
+    assert int(meta.cpu().numpy()[0]) == 0  # the Adler-32 sums of every kernel included
+    assert out.cpu().numpy().tobytes() == raw
+
+
+@pytest.mark.parametrize("skew", [1, 2, 3])
+def test_resolved_output_unaligned(gpu, skew):
+    """An output that starts between dwords; the bytes around it stay as they were."""
+    import ctypes
+    import torch
+    from cuda_zlib import _native
+    raw = _content("text", 3 * STRIPE + 5)
+    payload = zlib.compress(raw, 6)
+    lib = _native.load()
+    src = torch.from_numpy(np.frombuffer(payload, np.uint8).copy()).to(gpu)
+    out = torch.full((len(raw) + 8,), 0xA5, dtype=torch.uint8, device=src.device)
+    meta = torch.zeros(2, dtype=torch.uint32, device=src.device)
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    _native.check(lib, lib.HipZlibDecompress(
+        stream, 262144, 262144, ctypes.c_void_p(src.data_ptr()), len(payload),
+        ctypes.c_void_p(out.data_ptr() + skew), len(raw), ctypes.c_void_p(meta.data_ptr()), 2))
+    got = out.cpu().numpy()
+    assert int(meta.cpu().numpy()[0]) == 0
+    assert got[skew:skew + len(raw)].tobytes() == raw
+    assert (got[:skew] == 0xA5).all() and (got[skew + len(raw):] == 0xA5).all()
+
+
+def test_resolved_output_behind_dictionary(gpu):
+    import cuda_zlib
+    zdict = _content("text", 32768)
+    raw = zdict[1000:30000] + _content("text", 2 * STRIPE + 7)
+    c = zlib.compressobj(6, zlib.DEFLATED, -15, 8, zlib.Z_DEFAULT_STRATEGY, zdict)
+    payload = c.compress(raw) + c.flush()
+    out = cuda_zlib.decompress_deflate_raw(payload, len(raw), gpu, zdict=zdict)
+    assert out.cpu().numpy().tobytes() == raw
+
+
+def test_resolved_batch(gpu):
+    """Files whose edges fall inside tiles and stripes of the batch output."""
+    import cuda_zlib
+    sizes = [33, 4095, 65535, 1, 30001, 65536, 12345, 50000]
+    raws = [_content(("text", "period", "runs", "sparse")[i % 4] if n > 2000 else "text", n)
+            for i, n in enumerate(sizes)]
+    outs = cuda_zlib.decompress_zlib_batch([zlib.compress(r, 9) for r in raws], sizes, gpu)
+    for out, raw in zip(outs, raws):
+        assert out.cpu().numpy().tobytes() == raw
