@@ -1107,7 +1107,7 @@ __host__ __device__ __forceinline__ u32 crc_byte_update(u32 c, u32 byte) {
 }
 
 // a * b mod P over GF(2), both in the reflected representation.
-__host__ __device__ inline u32 crc_mul(u32 a, u32 b) {
+__host__ __device__ constexpr u32 crc_mul(u32 a, u32 b) {
   u32 p = 0;
   for (u32 i = 0; i < 32; ++i) {
     if ((a >> (31 - i)) & 1u) p ^= b;
@@ -1117,7 +1117,7 @@ __host__ __device__ inline u32 crc_mul(u32 a, u32 b) {
 }
 
 // x^(8n) mod P: the factor that appends n bytes after a register value.
-__host__ __device__ inline u32 crc_shift_bytes(u64 n) {
+__host__ __device__ constexpr u32 crc_shift_bytes(u64 n) {
   u32 r = 1u << 31;   // x^0
   u32 f = 1u << 23;   // x^8
   while (n) {

@@ -5088,15 +5088,24 @@ __global__ __launch_bounds__(kRestThreads) void g_resolve_rest(const State* st, 
 
 constexpr u32 kCrcTile = 16384;  // output bytes per CRC-32 tile (256 threads x 64)
 
-// CRC-32 registers (computed from 0, no inversions) of the 16 KiB tiles of
-// out[0..n), one workgroup per tile (grid-stride).  The last tile is read
-// right-aligned behind zero bytes: leading zeros leave a register that starts
-// at 0 unchanged, so every thread's 64-byte piece has full length and the
-// pieces join with one factor per tree level (x^(8 * 64 * 2^l)).
+// x^(8 * 64 * 2^l): the factors that join the pieces of a tile, then x^(8 * 2^14).
+struct CrcFactors {
+  u32 f[9];
+  constexpr CrcFactors() : f{} {
+    f[0] = crc_shift_bytes(64);
+    for (u32 l = 1; l < 9; ++l) f[l] = crc_mul(f[l - 1], f[l - 1]);
+  }
+};
+constexpr CrcFactors kCrcFactors;
+
+// CRC-32 registers of the 16 KiB tiles of out[0..n), one workgroup per tile
+// (grid-stride).  The register starts at all ones, which is the message's
+// first four bytes inverted, and the last tile ends with zero bytes up to its
+// full length (g_finish moves the expected value past them instead), so every
+// piece is full and every join factor a constant.
 __global__ __launch_bounds__(256) void g_crc_tiles(const State* st, const u8* out, u64 n,
                                                    u64* parts, u64 tiles, u32 open) {
   __shared__ u32 table[256];
-  __shared__ u32 factor[8];
   __shared__ u32 red[256];
   if (st->status || st->emit_status) return;
   if (open) {  // an open-ended decode's output is the bytes its path produced
@@ -5105,16 +5114,12 @@ __global__ __launch_bounds__(256) void g_crc_tiles(const State* st, const u8* ou
   }
   const u32 t = threadIdx.x;
   table[t] = crc_byte_update(0, t);
-  if (t < 8) factor[t] = crc_shift_bytes(u64(64) << t);
   __syncthreads();
   for (u64 tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
-    const u64 begin = tile * kCrcTile;
-    const u64 m = min<u64>(kCrcTile, n - begin);
-    const u64 pad = kCrcTile - m;
-    const u64 lo = u64(t) * 64;  // this thread's piece in the padded tile
-    u32 c = 0;
-    const u8* src = out + begin + lo;
-    if (!pad && (reinterpret_cast<uintptr_t>(src) & 15u) == 0) {
+    const u64 lo = tile * kCrcTile + u64(t) * 64;  // this thread's piece
+    u32 c = lo ? 0u : 0xffffffffu;
+    const u8* src = out + lo;
+    if (lo + 64 <= n && (reinterpret_cast<uintptr_t>(src) & 15u) == 0) {
       const uint4* v = reinterpret_cast<const uint4*>(src);
       uint4 q[4] = {v[0], v[1], v[2], v[3]};
       const u32* w = reinterpret_cast<const u32*>(q);
@@ -5122,16 +5127,16 @@ __global__ __launch_bounds__(256) void g_crc_tiles(const State* st, const u8* ou
         for (u32 k = 0; k < 4; ++k) c = table[(c ^ (w[j] >> (8 * k))) & 0xffu] ^ (c >> 8);
     } else {
       for (u32 j = 0; j < 64; ++j) {
-        const u64 p = lo + j;
-        const u32 b = p >= pad ? out[begin + p - pad] : 0u;
+        const u32 b = lo + j < n ? out[lo + j] : 0u;
         c = table[(c ^ b) & 0xffu] ^ (c >> 8);
       }
     }
     red[t] = c;
     __syncthreads();
+#pragma unroll
     for (u32 l = 0; l < 8; ++l) {
       const u32 w = 1u << l;
-      if ((t & (2 * w - 1)) == 0) red[t] = crc_mul(red[t], factor[l]) ^ red[t + w];
+      if ((t & (2 * w - 1)) == 0) red[t] = crc_mul(red[t], kCrcFactors.f[l]) ^ red[t + w];
       __syncthreads();
     }
     if (!t) parts[tile] = red[0];
@@ -5139,35 +5144,38 @@ __global__ __launch_bounds__(256) void g_crc_tiles(const State* st, const u8* ou
   }
 }
 
-// CRC-32 of out[0..n) from g_crc_tiles' registers, by one 256-thread
-// workgroup: each thread joins a run of tiles, then the runs join pairwise.
-// Valid in thread 0.
-__device__ u32 crc_from_tiles(const u64* parts, u64 n) {
+// Whether out[0..n), whose tile registers g_crc_tiles wrote, has the CRC-32
+// `wanted`, by one 256-thread workgroup (valid in thread 0).  Each thread joins
+// a run of tiles (the first runs start before the first tile, with zero
+// registers, so that all have one length), then the runs join pairwise; the
+// last wave meanwhile moves the wanted register past the padding of the last
+// tile.  (One join factor per run computed from its length by square and
+// multiply took 160 us of a 5 MB file; squared from level to level, 24 us.)
+__device__ bool crc_from_tiles(const u64* parts, u64 n, u32 wanted) {
   __shared__ u32 reg[256];
-  __shared__ u64 len[256];
+  __shared__ u32 moved;
+  if (!n) return !wanted;  // uniform
   const u32 t = threadIdx.x;
   const u64 tiles = (n + kCrcTile - 1) / kCrcTile;
-  const u64 per = (tiles + 255) / 256;
-  const u64 lo = min<u64>(tiles, t * per), hi = min<u64>(tiles, lo + per);
-  const u32 full = crc_shift_bytes(kCrcTile);
+  const u64 per = (tiles + 255) / 256, lead = 256 * per - tiles;
+  const u32 full = kCrcFactors.f[8];
   u32 c = 0;
-  u64 bytes = 0;
-  for (u64 k = lo; k < hi; ++k) {
-    const u64 m = min<u64>(kCrcTile, n - k * kCrcTile);
-    c = crc_mul(c, m == kCrcTile ? full : crc_shift_bytes(m)) ^ u32(parts[k]);
-    bytes += m;
+  for (u64 k = max(t * per, lead); k < (t + 1) * per; ++k)
+    c = crc_mul(c, full) ^ u32(parts[k - lead]);
+  u32 factor = full;  // full ^ per, by square and multiply
+  for (u32 b = 62u - u32(__clzll(per)); per > 1 && b < 64; --b) {
+    factor = crc_mul(factor, factor);
+    if ((per >> b) & 1u) factor = crc_mul(factor, full);
   }
   reg[t] = c;
-  len[t] = bytes;
+  if (t == 255) moved = crc_mul(~wanted, crc_shift_bytes(tiles * kCrcTile - n));
   __syncthreads();
   for (u32 w = 1; w < 256; w <<= 1) {
-    if ((t & (2 * w - 1)) == 0) {
-      reg[t] = crc_mul(reg[t], crc_shift_bytes(len[t + w])) ^ reg[t + w];
-      len[t] += len[t + w];
-    }
+    if ((t & (2 * w - 1)) == 0) reg[t] = crc_mul(reg[t], factor) ^ reg[t + w];
+    factor = crc_mul(factor, factor);
     __syncthreads();
   }
-  return crc_finish(reg[0], n);
+  return reg[0] == moved;
 }
 
 // Final status and the output on failure, over a grid of 256-thread
@@ -5212,8 +5220,8 @@ __global__ __launch_bounds__(256) void g_finish(State* st, u64 n, u32* meta, con
     }
   }
   if (!status && check == kCheckCrc) {  // uniform
-    const u32 got = crc_from_tiles(parts, n);
-    if (!t && (got != wanted || u32(n) != isize)) status = kGzipCheckMismatch;
+    const bool same = crc_from_tiles(parts, n, wanted);
+    if (!t && (!same || u32(n) != isize)) status = kGzipCheckMismatch;
   }
   if (!status && check == kCheckAdler) {  // uniform: every emitter and round wrote its pair
     u64 s = 0, w = 0;
