@@ -1503,14 +1503,7 @@ hipError_t run_deflate(hipStream_t stream, Scratch& scratch, const u8* in, u64 i
 }
 
 u64 deflate_scratch_bytes(u64 in_size, u32 chunk_bytes) {
-  struct Sizing final : Scratch {
-    u64 total = 0;
-    hipError_t alloc_bytes(void** p, u64 bytes) override {
-      *p = nullptr;
-      total += scratch_round(bytes);
-      return hipSuccess;
-    }
-  } sizing;
+  SizingScratch sizing;
   const u64 chunks = in_size ? (in_size + chunk_bytes - 1) / chunk_bytes : 1;
   ChunkBuffers b;
   (void)alloc_chunks(sizing, chunks, 1, in_size, b);

@@ -74,8 +74,7 @@ struct State {
   u64 fix_regions;
   u64 fix_runs;
   u64 fix_rt;
-  u64 fix_tasks;  // remainder tasks queued by the summary pass
-  u64 emit_units;  // emission units of long fixed runs queued for the unit pass
+    u64 emit_units;  // emission units of long fixed runs queued for the unit pass
 };
 
 // An open-ended decode's stream may end before the input does (other members
@@ -709,7 +708,6 @@ __global__ __launch_bounds__(256) void g_frame(const u8* in, u64 in_size, u32 fo
   st->fix_regions = 0;
   st->fix_runs = 0;
   st->fix_rt = 0;
-  st->fix_tasks = 0;
   st->emit_units = 0;
 }
 
@@ -1433,29 +1431,29 @@ __device__ u32 describe_block(BitIn& r, DecodeTables& t, u64 limit, u32& final_b
 // and a run of fixed blocks (Z_FIXED data, a text segment of the stress
 // stream) would otherwise belong to the segment of the candidate before it and
 // be described by one workgroup.  Instead describe defers such a run (a
-// "region"), and three passes decode it across the whole GPU:
-//   summaries  every 2 KiB tile of the region, from each of the 32 bit
+// "region"), and passes over it decode it across the whole GPU:
+//   summaries  every 1 KiB tile of the region, from each of the 32 bit
 //              offsets at which the tile's first token can start (a fixed
 //              token is at most 31 bits): where decoding leaves the tile,
-//              bytes produced, headers crossed, first EOB, or how it ended
+//              bytes produced, headers crossed, first EOB, or how it ended;
+//              then of groups of 64 tiles, for the walk
 //   walk       one wave per region chains the summaries from the run's first
 //              token (stored blocks between runs parsed in place), giving the
-//              true entry and output offset of every tile, the segment's end
-//              and block records; a tile without a summary is decoded there
-//   slices     every tile on a run decodes once more from its true entry to
-//              place the 512-bit emission slices inside it
+//              true entry and output offset of every tile or group, the
+//              segment's end and block records; a tile without a summary is
+//              decoded there
+//   slices     every tile on a run is decoded once more, and its slice
+//              summaries followed from its true entry place the 512-bit
+//              emission slices inside it
 // Emission then decodes a run's slices like a block's, crossing the fixed
 // headers inside a slice.  The reference keeps per-2 KiB-tile summaries of 32
 // entries for its serial chain walk (FixedSummary, scan_fixed_region,
 // _decode_kernels.py:376-472, 1181-1207, 1274).
-constexpr u32 kFixTileBits = 16384;
+constexpr u32 kFixTileBits = 8192;
 constexpr u32 kFixEntries = 32;
 constexpr u32 kFixSliceBits = 512;
 constexpr u32 kFixTileSlices = kFixTileBits / kFixSliceBits;
-constexpr u32 kFixProbeTokens = 512;  // tokens a fixed block is probed before it is deferred
-constexpr u32 kFixSyncBits = 256;     // entries decoded apart before those that meet share a task
-constexpr u32 kFixMarginBytes = 64;   // staged past a tile: its last token, an EOB and a header
-constexpr u32 kFixStageWords = (2 * kFixTileBits / 8 + kFixMarginBytes) / 4 + 4;
+constexpr u32 kFixProbeTokens = 128;  // tokens a fixed block is probed before it is deferred
 enum : u32 { kFixGo = 0, kFixEnd = 1, kFixHeader = 2, kFixError = 3 };
 constexpr u32 kFixInFinal = 0x10;       // kind flag: the exit lies inside the final block
 constexpr u16 kFixNoEob = 0xffffu;
@@ -1477,27 +1475,19 @@ struct FixSummary {
 };
 static_assert(sizeof(FixSummary) == 16, "summary layout");
 
-// The rest of one tile for the entries whose decodes reached the same token
-// start `p` (tile-relative, at or after kFixSyncBits) in the same state.
-struct FixTask {
-  u64 tile;
-  u32 entries;  // bit e: entry e
-  u16 p;
-  u16 in_final;
-};
-static_assert(sizeof(FixTask) == 16, "task layout");
-
 // A decode's summary from its prefix p (which ended, kind kFixGo, where r
-// starts) and the rest r.
+// starts) and the rest r, summarised as starting outside the final block: in
+// it, r's first EOB ends the stream.
 __device__ __forceinline__ FixSummary fix_join(const FixSummary& p, const FixSummary& r) {
   FixSummary s;
   const bool had_eob = p.eob != kFixNoEob;
-  s.bytes = p.bytes + r.bytes;
+  const bool fin = (p.kind & kFixInFinal) != 0, ends = fin && r.eob != kFixNoEob;
+  s.bytes = p.bytes + (ends ? r.eob_bytes : r.bytes);
   s.eob_bytes = had_eob ? p.eob_bytes : p.bytes + r.eob_bytes;
-  s.exit = r.exit;
+  s.exit = ends ? r.eob : r.exit;
   s.eob = had_eob ? p.eob : r.eob;
-  s.blocks = u16(p.blocks + r.blocks);
-  s.kind = r.kind;
+  s.blocks = u16(p.blocks + (ends ? 0 : r.blocks));
+  s.kind = ends ? u8(kFixEnd) : fin && r.kind == kFixGo ? u8(kFixGo | kFixInFinal) : r.kind;
   s.status = r.status;
   return s;
 }
@@ -1511,10 +1501,11 @@ struct FixRun {
   u64 b0;
   u32 lanes;
   u32 group;    // first of the run's consecutive slice groups
+  u64 size;     // output bytes
 };
 
 // Tiles k .. k + tiles - 1 of a run: the first one's true entry and the
-// run's output bytes before it (the others' follow from the summaries).
+// run's output bytes before it (g_fix_expand gives the others').
 struct FixTile {
   u64 pos;
   u32 off;
@@ -1523,10 +1514,12 @@ struct FixTile {
   u32 tiles;  // 1, or a group's tiles walked in one step
 };
 
-// The walk's step over a group of kFixGroupTiles marked tiles from one entry
-// state (entry bit e < 32 of the group's first tile, in the final block or
-// not): the tile summaries composed.
-constexpr u32 kFixGroupTiles = 16;
+// The walk's step from a tile to the end of its group of kFixGroupTiles marked
+// tiles, from one entry state (entry bit e < 32 of the tile, in the final
+// block or not): the tile summaries composed.  Kept for every kFixGroupEvery-th
+// tile of a group, so that a run which starts inside a group soon steps to its
+// end.
+constexpr u32 kFixGroupTiles = 64, kFixGroupEvery = 8;
 struct FixGroupSum {
   u32 bytes;   // output bytes up to the group's end or its terminal
   u32 blocks;  // block headers crossed
@@ -1547,41 +1540,6 @@ struct FixPeek {
     const u64 x0 = i < n ? w[i] : 0u, x1 = i + 1 < n ? w[i + 1] : 0u, x2 = i + 2 < n ? w[i + 2] : 0u;
     const u64 lo = x0 | (x1 << 32);
     return sh ? (lo >> sh) | (x2 << (64 - sh)) : lo;
-  }
-};
-
-// 64 bits at bit p of words in memory for one thread's forward decode: 128
-// bits in registers and the next 64 in flight, loaded when the position
-// moves past the first 64 (so a load has a few tokens of decoding to arrive).
-// Positions must not decrease by more than the window or jump more than 64
-// bits past it without a reload, which seek() does.  Words past `n` read as
-// zero.
-struct FixStream {
-  const u32* w;
-  u32 n;
-  u32 i0;  // even word index of `cur`
-  u64 cur, nxt, pend;
-  __device__ __forceinline__ u64 pair(u32 i) const {
-    return u64(i < n ? w[i] : 0u) | (u64(i + 1 < n ? w[i + 1] : 0u) << 32);
-  }
-  __device__ __forceinline__ void seek(u32 p) {
-    i0 = (p >> 5) & ~1u;
-    cur = pair(i0);
-    nxt = pair(i0 + 2);
-    pend = pair(i0 + 4);
-  }
-  __device__ __forceinline__ u64 operator()(u32 p) {
-    const u32 at = p - i0 * 32u;  // wraps when p precedes the window
-    if (at >= 128) {
-      seek(p);
-    } else if (at >= 64) {
-      cur = nxt;
-      nxt = pend;
-      i0 += 2;
-      pend = pair(i0 + 4);
-    }
-    const u32 sh = p - i0 * 32u;
-    return sh ? (cur >> sh) | (nxt << (64 - sh)) : cur;
   }
 };
 
@@ -2635,7 +2593,10 @@ __global__ __launch_bounds__(256) void g_fix_mark(const State* st, const u64* ca
         break;
       }
     }
-    if (tiles) fix_mark_tiles(fix_need, x / kFixTileBits, min<u64>(h / kFixTileBits, tiles - 1));
+    // To the end of its group, so that the walk takes the run's end in one step.
+    const u64 last = (h / kFixTileBits) | (kFixGroupTiles - 1);
+    if (tiles) fix_mark_tiles(fix_need, x / kFixTileBits / kFixGroupTiles * kFixGroupTiles,
+                              min<u64>(last, tiles - 1));
   }
 }
 
@@ -2647,184 +2608,316 @@ __device__ __forceinline__ u64 wave_fetch_add(u64* p, u64 v) {
   return __shfl(old, 0, 64);
 }
 
-// One wave's tile pair for g_fix_sum.  Every entry decodes to the first token
-// start at or after kFixSyncBits; entries that reach the same one in the same
-// state decode the same rest of the tile, which the lowest of them queues as
-// one task for g_fix_rem (with the queue full, each entry decodes it here).
-// The summaries of queued entries hold their prefixes until g_fix_rem joins
-// the rest.  Fixed codes resynchronize slowly: after 256 bits the 32 entries
-// of a tile typically still follow one to three token paths.
-__device__ void fix_sum_pair(const u8* body, u64 len, const u32* need, FixSummary* sum, u64 tiles,
-                             u64 k0, u32 pair, u32* w, u32 lane, State* st, FixTask* tasks,
-                             u64 task_capacity) {
-  // The wave stages body bits [k0 T, (k0 + 2) T) and the margin.
-  const uintptr_t base = reinterpret_cast<uintptr_t>(body);
-  const u64 byte0 = k0 * (kFixTileBits / 8);
-  const u64 first_word = (base + byte0) >> 2;
-  u64 last_byte = byte0 + 2 * (kFixTileBits / 8) + kFixMarginBytes;
-  if (last_byte > len) last_byte = len;
-  const u64 end_word = (base + last_byte + 3) >> 2;
-  const u32 nwords = u32(min<u64>(end_word > first_word ? end_word - first_word : 0, kFixStageWords));
-  const u32* g = reinterpret_cast<const u32*>(first_word << 2);
-  wave_sync();  // the previous pair's reads of the stage are done
-  for (u32 i = lane; i < nwords; i += 64) w[i] = g[i];
-  wave_sync();
-  const u32 half = lane >> 5, e = lane & 31u;
-  const u64 k = k0 + half;
-  const bool mine = k < tiles && ((pair >> half) & 1u);
-  const u32 skew = u32((base + byte0) & 3u) * 8;  // stage bit of body bit k0 T
-  const u32 rel = skew + half * kFixTileBits;
-  const u32 body_end = u32(min<u64>(len * 8 - k0 * kFixTileBits + skew, 0xffffffffull));
-  const FixPeek pk{w, nwords};
-  FixSummary f{};
-  if (mine) f = fix_scan(pk, rel + e, rel + kFixSyncBits, body_end, false, rel);
-  const bool go = mine && (f.kind & 15u) == kFixGo;
-  const u32 key = go ? u32(f.exit) | ((f.kind & kFixInFinal) ? 1u << 16 : 0u) | (half << 17) : ~0u;
-  // Each lane's representative: the lowest lane with its key.
-  u32 rep = lane, entries = 0;
-  for (u64 todo = __ballot(go); todo;) {
-    const u32 l = u32(__builtin_ctzll(todo));
-    const u32 kl = __shfl(key, int(l), 64);
-    const u64 same = __ballot(key == kl);
-    todo &= ~same;
-    if (key == kl) rep = l;
-    if (lane == l) entries = u32(same >> (32 * half));
+// ---- one tile's decodes, by one workgroup ---------------------------------------
+// Every bit position of the tile is decoded once, independently (thread t: the
+// 32 positions from bit 32 t, out of registers), into a 16-bit step; the
+// decodes of the 32 entries of each of the tile's 512-bit slices are then
+// chains of LDS reads over the steps, at most 73 long.
+//   step: twice the bits taken | the output bytes << 6 for a token; no bits for
+//   a special, whose value is kStepEob | the next header's three bits (| 8 if
+//   they are cut off) or an error's status.
+// Both parts are bound by VALU issue, so a position costs no branch and a link
+// of a chain four instructions (a first form, with branches and an unpacked
+// sum, took 1.7 times as long).
+// Measured on one MI355X, 15 MiB of Z_FIXED text: one thread per entry decoding
+// to bit 256 and one per distinct rest of a 2 KiB tile took 54 + 1080 us (a
+// token costs a thread of a nearly empty chip about 0.5 us), placing the
+// slices by one thread per tile 1210 us; this form 236 and 265 us.
+constexpr u32 kFixThreads = 256;
+constexpr u32 kStepEob = 16;
+static_assert(kFixThreads * 32 == kFixTileBits, "a thread decodes 32 positions");
+static_assert(kFixTileSlices * kFixEntries == 2 * kFixThreads, "two slice chains a thread");
+
+struct FixTileShared {
+  // Of the next 9 bits: where the length's extra bits start (bits 0-4), their
+  // number (5-9), the bits before a distance (10-14), the length's base
+  // (15-23), a distance follows (31).  An EOB takes the header's bits for
+  // extra ones.
+  u32 lut[512];
+  union {
+    __align__(16) u16 step[kFixTileBits];
+    FixSummary slice[kFixTileSlices][kFixEntries];  // of the slice's entries, relative to the tile
+  };
+};
+
+__device__ __forceinline__ void fix_build_lut(u32* lut) {
+  for (u32 i = threadIdx.x; i < 512; i += blockDim.x) {
+    const u32 r9 = __builtin_bitreverse32(i) >> 23;
+    u32 sym, l;
+    if ((r9 >> 2) < 24) {
+      sym = 256 + (r9 >> 2);
+      l = 7;
+    } else if ((r9 >> 1) < 0xC8) {
+      sym = (r9 >> 1) < 0xC0 ? (r9 >> 1) - 0x30 : (r9 >> 1) + 88;  // 0xC0 -> 280
+      l = 8;
+    } else {
+      sym = r9 - 256;
+      l = 9;
+    }
+    u32 v = (l << 10) | (1u << 15);  // a literal
+    if (sym == 256) {
+      v = 7u | (3u << 5) | (kStepEob << 15);
+    } else if (sym > 285) {
+      v = u32(kBadSymbol) << 15;
+    } else if (sym > 256) {
+      const u32 x = length_extra(sym - 257);
+      v = l | (x << 5) | ((l + x) << 10) | (length_base(sym - 257) << 15) | 0x80000000u;
+    }
+    lut[i] = v;
   }
-  const bool lead = go && rep == lane;
-  const u64 leads = __ballot(lead);
-  const u64 slot0 = leads ? wave_fetch_add(&st->fix_tasks, u64(__popcll(leads))) : 0;
-  const u64 slot = slot0 + u64(__popcll(leads & ((1ull << lane) - 1)));
-  const bool queued = lead && slot < task_capacity;
-  if (queued) {
-    FixTask tk;
-    tk.tile = k;
-    tk.entries = entries;
-    tk.p = f.exit;
-    tk.in_final = (f.kind & kFixInFinal) ? 1 : 0;
-    tasks[slot] = tk;
+}
+
+// The steps of tile k's positions from bit 32 t.  `end`: the body's end
+// relative to the tile (a step that passes it is an error), unchecked when it
+// lies past every step.
+template <bool kEnd>
+__device__ __forceinline__ void fix_steps(const u8* body, u64 len, u64 k, u32 end, u32 t,
+                                          const u32* lut, u16* step) {
+  const uintptr_t at = reinterpret_cast<uintptr_t>(body) + k * (kFixTileBits / 8);
+  const u32* w = reinterpret_cast<const u32*>(at & ~uintptr_t(3)) + t;
+  const u32* stop = reinterpret_cast<const u32*>((reinterpret_cast<uintptr_t>(body) + len + 3) &
+                                                 ~uintptr_t(3));
+  const u32 skew = u32(at & 3u) * 8;
+  const u32 x0 = w < stop ? w[0] : 0u, x1 = w + 1 < stop ? w[1] : 0u, x2 = w + 2 < stop ? w[2] : 0u;
+  const u32 a0 = __builtin_amdgcn_alignbit(x1, x0, skew), a1 = __builtin_amdgcn_alignbit(x2, x1, skew);
+#pragma unroll
+  for (u32 i8 = 0; i8 < 32; i8 += 8) {
+    u32 o[8];
+#pragma unroll
+    for (u32 j = 0; j < 8; ++j) {
+      const u32 i = i8 + j;
+      const u32 b = __builtin_amdgcn_alignbit(a1, a0, i);
+      const u32 v = lut[b & 511u];
+      const u32 value = __builtin_amdgcn_ubfe(v, 15, 9) + __builtin_amdgcn_ubfe(b, v, v >> 5);
+      const u32 lx = __builtin_amdgcn_ubfe(v, 10, 5);
+      const u32 d = __builtin_bitreverse32(b >> lx) >> 27;  // the distance symbol
+      const u32 follows = u32(i32(v) >> 31);
+      const u32 nb = lx + ((max(d >> 1, 1u) + 4u) & follows);
+      u32 r = (nb << 1) | (value << 6);
+      if ((d & follows) > 29) r = u32(kBadSymbol) << 6;
+      if (kEnd) {
+        const u32 p = 32 * t + i;
+        const bool eob = (r & 63u) == 0 && (value & kStepEob), token = (r & 63u) != 0;
+        if ((token && p + nb > end) || (eob && p + 7 > end)) r = u32(kTruncated) << 6;
+        else if (eob && p + 10 > end) r |= 8u << 6;
+      }
+      o[j] = r;
+    }
+    *reinterpret_cast<uint4*>(step + 32 * t + i8) =
+        make_uint4(o[0] | (o[1] << 16), o[2] | (o[3] << 16), o[4] | (o[5] << 16), o[6] | (o[7] << 16));
   }
-  const u64 taken = __ballot(queued);
-  if (go && !((taken >> rep) & 1u))
-    f = fix_join(f, fix_scan(pk, rel + f.exit, rel + kFixTileBits, body_end,
-                             (f.kind & kFixInFinal) != 0, rel));
-  if (mine) sum[k * kFixEntries + e] = f;
+}
+
+// The decode from p to the first token start at or after `stop` (both inside
+// the tile), outside the final block, over the steps: as fix_scan.
+__device__ __forceinline__ FixSummary fix_chain(const u16* step, u32 p, u32 stop) {
+  FixSummary s;
+  s.bytes = 0;
+  s.eob_bytes = 0;
+  s.eob = kFixNoEob;
+  s.blocks = 0;
+  s.status = 0;
+  u32 kind = kFixGo, bytes = 0;
+  bool in_final = false;
+  while (p < stop) {
+    // Tokens: the steps' sum less the bits moved is the bytes' sum.
+    const u32 p2 = 2 * p;
+    u32 q = p2, sum = 0, v, nb;
+    do {
+      v = *reinterpret_cast<const u16*>(reinterpret_cast<const u8*>(step) + q);
+      nb = v & 63u;
+      sum += v;
+      q += nb;
+    } while (nb && q < 2 * stop);
+    if (!nb) sum -= v;
+    bytes += (sum - (q - p2)) >> 6;
+    p = q >> 1;
+    if (nb) break;
+    const u32 value = v >> 6;
+    if (!(value & kStepEob)) {
+      kind = kFixError;
+      s.status = u8(value);
+      break;
+    }
+    p += 7;
+    if (s.eob == kFixNoEob) {
+      s.eob = u16(p);
+      s.eob_bytes = bytes;
+    }
+    if (in_final) {
+      kind = kFixEnd;
+      break;
+    }
+    if (value & 8u) {
+      kind = kFixError;
+      s.status = kTruncated;
+      break;
+    }
+    if (((value >> 1) & 3u) != 1u) {
+      kind = kFixHeader;
+      break;
+    }
+    ++s.blocks;
+    in_final = value & 1u;
+    p += 3;
+  }
+  s.bytes = bytes;
+  s.exit = u16(p);
+  s.kind = u8(kind | (kind == kFixGo && in_final ? kFixInFinal : 0u));
+  return s;
+}
+
+// Tile k's slice summaries into sh.slice (the LUT is built).  `from` below
+// the tile's end: `first` gets the decode from that position to the end of
+// its slice (thread 0).
+__device__ __forceinline__ void fix_tile(const u8* body, u64 len, u64 k, FixTileShared& sh,
+                                         u32 from, FixSummary& first) {
+  const u32 t = threadIdx.x;
+  const u64 rest = len * 8 - k * kFixTileBits;
+  if (rest >= kFixTileBits + 64) fix_steps<false>(body, len, k, 0, t, sh.lut, sh.step);
+  else fix_steps<true>(body, len, k, u32(rest), t, sh.lut, sh.step);
+  lds_barrier();
+  FixSummary mine[2];
+#pragma unroll
+  for (u32 q = 0; q < 2; ++q) {
+    const u32 c = q * kFixThreads + t, s0 = c / kFixEntries * kFixSliceBits;
+    mine[q] = fix_chain(sh.step, s0 + c % kFixEntries, s0 + kFixSliceBits);
+  }
+  if (!t && from < kFixTileBits)
+    first = fix_chain(sh.step, from, (from / kFixSliceBits + 1) * kFixSliceBits);
+  lds_barrier();  // the summaries take the steps' place
+#pragma unroll
+  for (u32 q = 0; q < 2; ++q) (&sh.slice[0][0])[q * kFixThreads + t] = mine[q];
+  lds_barrier();
 }
 
 }  // namespace
 
-// Summaries of the marked tiles (one wave per two tiles: lane e decodes the
-// first tile from its entry bit e, lane 32 + e the second), over the tiles
-// and a margin staged in LDS.  Waves take tile pairs grid-stride.
-__global__ __launch_bounds__(256) void g_fix_sum(const u8* body, u64 len, State* st,
-                                                 const u32* need, FixSummary* sum, u64 tiles,
-                                                 FixTask* tasks, u64 task_capacity) {
-  __shared__ u32 words[kDescThreads / 64][kFixStageWords];
+// Summaries of the marked tiles: a workgroup per tile, grid-stride.  Each
+// entry's summary is its slices' summaries joined (a token start at or after a
+// slice's end is one of the next slice's entries: no token or header passes
+// 31 bits of it).
+__global__ __launch_bounds__(kFixThreads) void g_fix_sum(const u8* body, u64 len, const State* st,
+                                                         const u32* need, FixSummary* sum,
+                                                         u64 tiles) {
+  __shared__ FixTileShared sh;
   if (st->status || !st->fix_regions) return;
-  const u32 lane = lane_id(), wave = threadIdx.x >> 6;
-  const u64 waves = u64(gridDim.x) * (kDescThreads / 64);
-  for (u64 k0 = (u64(blockIdx.x) * (kDescThreads / 64) + wave) * 2; k0 < tiles; k0 += 2 * waves) {
-    const u32 pair = (need[k0 >> 5] >> (k0 & 31)) & 3u;  // k0 is even: one need word
-    if (pair)
-      fix_sum_pair(body, len, need, sum, tiles, k0, pair, words[wave], lane, st, tasks,
-                   task_capacity);
-  }
-}
-
-// The queued rests of tiles: one thread per task decodes from the task's
-// token start to the tile's end (the body read through the cache) and joins
-// the result to the summaries of the task's entries.
-__global__ __launch_bounds__(256) void g_fix_rem(const u8* body, u64 len, const State* st,
-                                                 const FixTask* tasks, u64 task_capacity,
-                                                 FixSummary* sum) {
-  if (st->status || !st->fix_regions) return;
-  const u64 n = min<u64>(st->fix_tasks, task_capacity);
-  const uintptr_t base = reinterpret_cast<uintptr_t>(body);
-  for (u64 i = u64(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
-       i += u64(gridDim.x) * blockDim.x) {
-    const FixTask tk = tasks[i];
-    // The tile and its margin, as g_fix_sum staged them.
-    const u64 byte0 = tk.tile * (kFixTileBits / 8);
-    const u64 first_word = (base + byte0) >> 2;
-    u64 last_byte = byte0 + kFixTileBits / 8 + kFixMarginBytes;
-    if (last_byte > len) last_byte = len;
-    const u64 end_word = (base + last_byte + 3) >> 2;
-    const u32 nwords = u32(end_word > first_word ? end_word - first_word : 0);
-    const u32 skew = u32((base + byte0) & 3u) * 8;
-    const u32 body_end = u32(min<u64>(len * 8 - tk.tile * kFixTileBits + skew, 0xffffffffull));
-    FixStream pk;
-    pk.w = reinterpret_cast<const u32*>(first_word << 2);
-    pk.n = nwords;
-    pk.seek(skew + tk.p);
-    const FixSummary r =
-        fix_scan(pk, skew + tk.p, skew + kFixTileBits, body_end, tk.in_final != 0, skew);
-    for (u32 m = tk.entries; m; m &= m - 1) {
-      FixSummary* s = sum + tk.tile * kFixEntries + __builtin_ctz(m);
-      *s = fix_join(*s, r);
+  fix_build_lut(sh.lut);
+  lds_barrier();
+  for (u64 k = blockIdx.x; k < tiles; k += gridDim.x) {
+    if (!((need[k >> 5] >> (k & 31)) & 1u)) continue;  // uniform
+    FixSummary f;
+    fix_tile(body, len, k, sh, kFixTileBits, f);
+    if (threadIdx.x < kFixEntries) {
+      f = sh.slice[0][threadIdx.x];
+      for (u32 s = 1; s < kFixTileSlices && (f.kind & 15u) == kFixGo; ++s)
+        f = fix_join(f, sh.slice[s][f.exit - s * kFixSliceBits]);
+      sum[k * kFixEntries + threadIdx.x] = f;
     }
+    lds_barrier();  // the next tile's steps take the summaries' place
   }
 }
 
-// Group summaries for the walk: one thread per (group of kFixGroupTiles
-// wholly marked tiles, entry state) composes the group's tile summaries as
-// the walk would step them (in the final block, a tile's first EOB ends the
-// stream).
+// Group summaries for the walk: a workgroup per group of kFixGroupTiles wholly
+// marked tiles stages the tiles' summaries, and a thread per entry state
+// composes them from the last tile back, as the walk would step them (in the
+// final block, a tile's first EOB ends the stream).
 __global__ __launch_bounds__(256) void g_fix_groups(const State* st, const u32* need,
                                                     const FixSummary* sum, u64 tiles,
                                                     FixGroupSum* groups) {
+  __shared__ FixSummary all[kFixGroupTiles][kFixEntries];
+  __shared__ FixGroupSum rest[64];  // from the tile after, by entry state
   if (st->status || !st->fix_regions) return;
-  const u64 n = tiles / kFixGroupTiles * 64;
-  for (u64 i = u64(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
-       i += u64(gridDim.x) * blockDim.x) {
-    const u64 k0 = i / 64 * kFixGroupTiles;
-    if (((need[k0 >> 5] >> (k0 & 31)) & 0xffffu) != 0xffffu) continue;  // stepped tile by tile
-    u32 e = u32(i & 31), bytes = 0, blocks = 0;
-    bool fin = (i & 32) != 0;
-    FixGroupSum r;
-    r.exit = 0;
-    r.kind = 0;
-    r.tiles = 0;
-    r.status = 0;
-    for (u32 j = 0; j < kFixGroupTiles; ++j) {
-      FixSummary f = sum[(k0 + j) * kFixEntries + e];
-      if (fin && f.eob != kFixNoEob) {
-        f.kind = kFixEnd;
-        f.exit = f.eob;
-        f.bytes = f.eob_bytes;
-        f.blocks = 0;
-      }
-      bytes += f.bytes;
-      blocks += f.blocks;
-      if ((f.kind & 15u) != kFixGo) {
+  for (u64 g = blockIdx.x; g < tiles / kFixGroupTiles; g += gridDim.x) {
+    const u64 k0 = g * kFixGroupTiles;
+    static_assert(kFixGroupTiles == 64, "a group's marks are two words");
+    if ((need[k0 >> 5] & need[(k0 >> 5) + 1]) != ~0u) continue;  // uniform: stepped tile by tile
+    const uint4* src = reinterpret_cast<const uint4*>(sum + k0 * kFixEntries);
+    for (u32 i = threadIdx.x; i < kFixGroupTiles * kFixEntries; i += 256)
+      reinterpret_cast<uint4*>(&all[0][0])[i] = src[i];
+    __syncthreads();
+    if (threadIdx.x < 64) {
+      const u32 e = threadIdx.x & 31u;
+      const bool fin = (threadIdx.x & 32) != 0;
+      for (u32 j = kFixGroupTiles; j-- > 0;) {
+        const FixSummary f = all[j][e];
+        FixGroupSum r;
+        r.bytes = f.bytes;
+        r.blocks = f.blocks;
         r.exit = f.exit;
         r.kind = f.kind;
-        r.tiles = u8(j + 1);
+        r.tiles = 1;
         r.status = f.status;
-        break;
+        if (fin && f.eob != kFixNoEob) {
+          r.bytes = f.eob_bytes;
+          r.blocks = 0;
+          r.exit = f.eob;
+          r.kind = kFixEnd;
+        } else if ((f.kind & 15u) == kFixGo) {
+          const bool in_final = fin || (f.kind & kFixInFinal) != 0;
+          r.kind = u8(kFixGo | (in_final ? kFixInFinal : 0u));
+          if (j + 1 < kFixGroupTiles) {
+            const FixGroupSum n = rest[(f.exit - kFixTileBits) + (in_final ? 32 : 0)];
+            r.bytes += n.bytes;
+            r.blocks += n.blocks;
+            r.exit = n.exit;
+            r.kind = n.kind;
+            r.tiles = u8(n.tiles + 1);
+            r.status = n.status;
+          }
+        }
+        wave_sync();
+        rest[threadIdx.x] = r;
+        wave_sync();
+        if (j % kFixGroupEvery == 0) groups[(k0 + j) / kFixGroupEvery * 64 + threadIdx.x] = r;
       }
-      fin = fin || (f.kind & kFixInFinal) != 0;
-      if (f.exit < kFixTileBits || f.exit - kFixTileBits >= kFixEntries) break;  // no jump (r.tiles 0)
-      if (j + 1 == kFixGroupTiles) {
-        r.exit = f.exit;
-        r.kind = u8(kFixGo | (fin ? kFixInFinal : 0u));
-        r.tiles = u8(kFixGroupTiles);
-      }
-      e = f.exit - kFixTileBits;
     }
-    r.bytes = bytes;
-    r.blocks = blocks;
-    groups[i] = r;
+    __syncthreads();
   }
 }
 
-
+// The true entries of the tiles a walk stepped over in groups: per slot of
+// more than one tile, the entry bit (low 5 bits of x) and the run's output
+// bytes before (y) of every tile after the first, at the tile's index.  A tile
+// lies in one such step only (a run that starts in a step's last tile enters
+// that tile past its 32 entry bits: a stored block lies between).
+__global__ __launch_bounds__(256) void g_fix_expand(const State* st, const FixTile* rt,
+                                                    u64 rt_capacity, const FixSummary* sum,
+                                                    uint2* entries) {
+  __shared__ FixSummary all[kFixGroupTiles][kFixEntries];
+  if (st->status || !st->fix_regions) return;
+  const u64 used = min<u64>(st->fix_rt, rt_capacity);
+  for (u64 i = blockIdx.x; i < used; i += gridDim.x) {
+    const FixTile ft = rt[i];
+    if (ft.run == kNone || ft.tiles < 2) continue;  // uniform
+    const uint4* src = reinterpret_cast<const uint4*>(sum + u64(ft.k) * kFixEntries);
+    for (u32 q = threadIdx.x; q < ft.tiles * kFixEntries; q += 256)
+      reinterpret_cast<uint4*>(&all[0][0])[q] = src[q];
+    __syncthreads();
+    if (threadIdx.x < 64) {
+      u32 e = u32(ft.pos - u64(ft.k) * kFixTileBits), off = ft.off;
+      uint2 mine = make_uint2(0, 0);
+      for (u32 j = 1; j < ft.tiles; ++j) {
+        const FixSummary f = all[j - 1][e & 31u];
+        off += f.bytes;
+        e = f.exit - kFixTileBits;
+        if (threadIdx.x == j) mine = make_uint2(e & 31u, off);
+      }
+      if (threadIdx.x && threadIdx.x < ft.tiles) entries[u64(ft.k) + threadIdx.x] = mine;
+    }
+    __syncthreads();
+  }
+}
 
 namespace {
 
-constexpr u32 kFixBatch = 16;  // tiles of summaries a walk holds in LDS at once
+constexpr u32 kFixBatch = 16;  // tiles (and groups) of summaries a walk holds in LDS at once
 
 struct FixWalkShared {
   FixSummary batch[kFixBatch][kFixEntries];
-  u32 words[kFixStageWords / 2 + 8];  // one tile and its margin, for decodes without a summary
+  FixGroupSum groups[kFixBatch][64];
+  u32 lut[512];         // for decodes without a summary: the tile's steps
+  __align__(16) u16 step[kFixTileBits];
 };
 
 // An atomic add by lane 0, its old value given to every lane.
@@ -2870,7 +2963,8 @@ __global__ __launch_bounds__(64) void g_fix_walk(
     u32 slot_used = 64;
     bool chunk = false;  // slots slot_base .. +63 are this walk's (unused ones marked at the end)
     FixTile mine;        // lane l: slot l of the chunk, stored when the chunk is done
-    u64 batch_k = ~0ull;
+    u64 batch_k = ~0ull, batch_g = ~0ull;
+    bool lut = false;  // sh.lut is built
     u64 need_at = ~0ull;  // index of the cached word of the tile marks
     u32 need_word = 0;
     // Finishes the open run at bit `e_end`: its record, slice groups and FixRun.
@@ -2893,6 +2987,7 @@ __global__ __launch_bounds__(64) void g_fix_walk(
         fr.b0 = b0;
         fr.lanes = u32(lanes);
         fr.group = u32(g);
+        fr.size = out - run_out0;
         runs[run_id] = fr;
         BlockRec rec;
         rec.start = run_hdr;
@@ -2999,15 +3094,32 @@ __global__ __launch_bounds__(64) void g_fix_walk(
         need_word = need[need_at];
       }
       const bool have = e < kFixEntries && k < tiles && ((need_word >> (k & 31)) & 1u);
-      // At the first tile of a group of marked tiles: the whole group in one
-      // step, unless the output or block limit fails inside it (then tile by
-      // tile, which finds the failing tile).
+      // In a group of marked tiles: to the group's end in one step, unless
+      // the output or block limit fails on the way (then tile by tile, which
+      // finds the failing tile).
       FixGroupSum gs;
       bool jump = false;
-      if (have && k % kFixGroupTiles == 0 && k + kFixGroupTiles <= tiles &&
-          ((need_word >> (k & 31)) & 0xffffu) == 0xffffu) {
-        gs = groups[k / kFixGroupTiles * 64 + e + (in_final ? 32 : 0)];
-        jump = gs.tiles != 0 && out + gs.bytes <= out_size && blocks + gs.blocks <= kMaxBlocks;
+      const u64 gk = k & ~u64(kFixGroupTiles - 1);
+      if (have && k % kFixGroupEvery == 0 && gk + kFixGroupTiles <= tiles &&
+          (need_word & need[need_at ^ 1]) == ~0u) {
+        const u32 state = e + (in_final ? 32 : 0);
+        if (k != gk) {
+          gs = groups[k / kFixGroupEvery * 64 + state];
+        } else {
+          const u64 g = k / kFixGroupTiles;
+          if (g < batch_g || g >= batch_g + kFixBatch) {
+            // The next kFixBatch groups' summaries, 16 bytes a load.
+            const u64 avail = min<u64>(kFixBatch, tiles / kFixGroupTiles - g);
+            constexpr u32 kStride = kFixGroupTiles / kFixGroupEvery * 64;
+            for (u32 i = 0; i < avail; ++i)
+              reinterpret_cast<uint4*>(&sh.groups[i][0])[lane] =
+                  reinterpret_cast<const uint4*>(groups + (g + i) * kStride)[lane];
+            wave_sync();
+            batch_g = g;
+          }
+          gs = sh.groups[g - batch_g][state];
+        }
+        jump = out + gs.bytes <= out_size && blocks + gs.blocks <= kMaxBlocks;
       }
       if (recs_ok && run_id != kNone) {
         if (slot_used == 64) {
@@ -3065,31 +3177,26 @@ __global__ __launch_bounds__(64) void g_fix_walk(
           batch_k = k;
         }
         f = sh.batch[k - batch_k][e];
-        if (in_final && f.eob != kFixNoEob) {
-          // The stream's last block ends at its first EOB.
-          f.kind = kFixEnd;
-          f.exit = f.eob;
-          f.bytes = f.eob_bytes;
-          f.blocks = 0;
-        }
       } else {
-        // Decode from the stage: tile k and its margin.
-        const u64 byte0 = k * (kFixTileBits / 8);
-        const u64 first_word = (base + byte0) >> 2;
-        u64 last_byte = byte0 + kFixTileBits / 8 + kFixMarginBytes;
-        if (last_byte > len) last_byte = len;
-        const u64 end_word = (base + last_byte + 3) >> 2;
-        const u32 nwords = u32(min<u64>(end_word > first_word ? end_word - first_word : 0,
-                                        kFixStageWords / 2 + 8));
-        const u32* gw = reinterpret_cast<const u32*>(first_word << 2);
-        wave_sync();  // earlier reads of the stage are done
-        for (u32 i = lane; i < nwords; i += 64) sh.words[i] = gw[i];
+        // The tile's steps by the wave, followed from pos (one thread over the
+        // staged bits took about 0.35 us a token, 160 us from mid-tile).
+        if (!lut) fix_build_lut(sh.lut);
+        lut = true;
+        wave_sync();  // and earlier reads of the steps are done
+        const u64 rest = len * 8 - k * kFixTileBits;
+        for (u32 t = lane; t < kFixTileBits / 32; t += 64) {
+          if (rest >= kFixTileBits + 64) fix_steps<false>(body, len, k, 0, t, sh.lut, sh.step);
+          else fix_steps<true>(body, len, k, u32(rest), t, sh.lut, sh.step);
+        }
         wave_sync();
-        const u32 skew = u32((base + byte0) & 3u) * 8;
-        const u64 body_end = len * 8 - k * kFixTileBits + skew;
-        const FixPeek pk{sh.words, nwords};
-        f = fix_scan(pk, skew + e, skew + kFixTileBits, u32(min<u64>(body_end, 0xffffffffull)),
-                     in_final, skew);
+        f = fix_chain(sh.step, e, kFixTileBits);
+      }
+      if (in_final && f.eob != kFixNoEob) {
+        // The stream's last block ends at its first EOB.
+        f.kind = kFixEnd;
+        f.exit = f.eob;
+        f.bytes = f.eob_bytes;
+        f.blocks = 0;
       }
       out += f.bytes;
       blocks += f.blocks;
@@ -3097,7 +3204,7 @@ __global__ __launch_bounds__(64) void g_fix_walk(
       if (blocks > kMaxBlocks) { status = kBlockCapacity; break; }
       const u32 kind = f.kind & 15u;
       if (kind == kFixGo) {
-        in_final = (f.kind & kFixInFinal) != 0 || (have && in_final);
+        in_final = (f.kind & kFixInFinal) != 0 || in_final;
         pos = k * kFixTileBits + f.exit;
       } else if (kind == kFixEnd) {
         pos = k * kFixTileBits + f.exit;
@@ -3131,84 +3238,67 @@ __global__ __launch_bounds__(64) void g_fix_walk(
   }
 }
 
-// Slices of the walked runs: one thread per tile slot decodes the tile from
-// its true entry and places the slices whose 512-bit windows start inside
-// it (slice b - b0 of the run starts at the first token at or after bit
-// 512 b; where the run ends first, at the run's end, with nothing to decode).
-__global__ __launch_bounds__(256) void g_fix_slices(const u8* body, u64 len, const State* st,
-                                                    const FixTile* rt, u64 rt_capacity,
-                                                    const FixRun* runs, u64 run_capacity,
-                                                    const FixSummary* sum, u64* slice_entry,
-                                                    u32* slice_off) {
+// Slices of the walked runs: a workgroup per tile (blockIdx.y: the tile within
+// its slot) decodes it as g_fix_sum does and follows the slice summaries from
+// the tile's true entry: slice b - b0 of the run starts at the first token at
+// or after bit 512 b; where the run ends first, at the run's end, with nothing
+// to decode.
+__global__ __launch_bounds__(kFixThreads) void g_fix_slices(const u8* body, u64 len,
+                                                            const State* st, const FixTile* rt,
+                                                            u64 rt_capacity, const FixRun* runs,
+                                                            u64 run_capacity, const uint2* entries,
+                                                            u64* slice_entry, u32* slice_off) {
+  __shared__ FixTileShared sh;
   if (st->status || !st->fix_regions) return;
   const u64 used = min<u64>(st->fix_rt, rt_capacity);
   const u64 nruns = min<u64>(st->fix_runs, run_capacity);
-  const uintptr_t base = reinterpret_cast<uintptr_t>(body);
-  const u32* words = reinterpret_cast<const u32*>(base & ~uintptr_t(3));
-  const u64 skew = u64(base & 3u) * 8;
-  const u64 nwords = (u64(base & 3u) + len + 3) / 4;
-  for (u64 i = u64(blockIdx.x) * blockDim.x + threadIdx.x; i < used * kFixGroupTiles;
-       i += u64(gridDim.x) * blockDim.x) {
-    // Tile j of slot i / kFixGroupTiles.
-    const FixTile ft = rt[i / kFixGroupTiles];
-    const u32 j = u32(i % kFixGroupTiles);
-    if (ft.run == kNone || ft.run >= nruns || j >= ft.tiles) continue;
+  bool built = false;
+  const auto tile = [&](const FixTile& ft, u32 j) {
     const FixRun run = runs[ft.run];
-    if (!run.lanes) continue;
-    // The tile's true entry and offset: through the summaries of the tiles
-    // before it in the group (inside a group every tile but the last is
-    // left at its end, so the final-block rule never applies to them).
-    const u64 k = u64(ft.k) + j;
-    u64 p = ft.pos;
-    u32 off = ft.off;
+    if (!run.lanes) return;
+    if (!built) fix_build_lut(sh.lut);
+    built = true;
+    lds_barrier();
+    const u64 k = u64(ft.k) + j, tile0 = k * kFixTileBits;
+    u32 p = u32(ft.pos - tile0), off = ft.off;
     if (j) {
-      u32 e = u32(ft.pos - u64(ft.k) * kFixTileBits);
-      for (u32 q = 0; q < j; ++q) {
-        const FixSummary f = sum[(u64(ft.k) + q) * kFixEntries + e];
+      const uint2 e = entries[k];
+      p = e.x;
+      off = e.y;
+    }
+    // A run starts anywhere in a tile; every later entry is a summary's.
+    const bool inside = p % kFixSliceBits >= kFixEntries;
+    FixSummary first;
+    fix_tile(body, len, k, sh, inside ? p : kFixTileBits, first);
+    if (!threadIdx.x) {
+      const u64 bl = run.b0 + run.lanes - 1;
+      const u64 at = u64(run.group) * 64 - run.b0;  // slice index of window b: at + b
+      bool ended = false;
+      for (u64 b = tile0 / kFixSliceBits + p / kFixSliceBits; b <= bl; ++b) {
+        const u32 s = u32(b - tile0 / kFixSliceBits);
+        if (s >= kFixTileSlices && !ended) break;  // the next tile places the rest
+        slice_entry[at + b] = ended ? run.end : tile0 + p;
+        slice_off[at + b] = ended ? u32(run.size) : off;
+        if (ended) continue;
+        const u32 e = p - s * kFixSliceBits;
+        const FixSummary f = e < kFixEntries ? sh.slice[s][e] : first;
         off += f.bytes;
-        e = u32(f.exit) - kFixTileBits;
+        p = f.exit;
+        ended = (f.kind & 15u) != kFixGo || tile0 + p >= run.end;
       }
-      p = k * kFixTileBits + e;
     }
-    const u64 bl = run.b0 + run.lanes - 1;
-    const u64 bf = max<u64>(run.b0, k * kFixTileSlices);
-    const u64 bt = min<u64>(bl, k * kFixTileSlices + kFixTileSlices - 1);
-    const u64 at = u64(run.group) * 64 - run.b0;  // slice index of window b: at + b
-    slice_entry[at + bf] = p;
-    slice_off[at + bf] = off;
-    // Windows up to bt; the tile whose decode reaches the run's end also
-    // places the windows after it (the run's last EOB may end past the tile).
-    const u64 tile_end = (k + 1) * kFixTileBits;
-    // The body read from the tile's first word on (bit p at p - tile + skew).
-    const u64 tile0 = k * kFixTileBits, w0 = tile0 / 32;
-    FixStream in;
-    in.w = words + w0;
-    in.n = u32(min<u64>(nwords > w0 ? nwords - w0 : 0, 0xffffffffull));
-    in.seek(u32(p - tile0 + skew));
-    for (u64 b = bf + 1; b <= bl;) {
-      if (p >= run.end || (b <= bt && p >= b * kFixSliceBits)) {
-        if (p > run.end) p = run.end;
-        slice_entry[at + b] = p;
-        slice_off[at + b] = off;
-        ++b;
-        continue;
-      }
-      if (b > bt && p >= tile_end) break;  // the next tile places the rest
-      // 64 body bits at p (bits past the body's words read as zero).
-      const u64 bits = in(u32(p - tile0 + skew));
-      u32 nb, length, value;
-      const u32 kind = fixed_token(bits, nb, length, value);
-      if (kind == kKindBad) {
-        p = run.end;  // never on a walked run; emission then reports an extent error
-        continue;
-      }
-      if (kind == kKindEob) {
-        p = p + 7 >= run.end ? run.end : p + 10;  // past the next fixed header
-        continue;
-      }
-      off += length;
-      p += nb;
-    }
+    lds_barrier();  // the next tile's steps take the summaries' place
+  };
+  // Tile blockIdx.y of the slots of many tiles, then the slots of one tile
+  // dealt over the whole grid.
+  for (u64 i = blockIdx.x; i < used; i += gridDim.x) {
+    const FixTile ft = rt[i];
+    if (ft.run < nruns && ft.tiles > 1 && blockIdx.y < ft.tiles) tile(ft, blockIdx.y);  // uniform
+  }
+  for (u64 i = blockIdx.x + u64(gridDim.x) * blockIdx.y; i < used;
+       i += u64(gridDim.x) * gridDim.y) {
+    const FixTile ft = rt[i];
+    if (ft.run < nruns && ft.tiles == 1) tile(ft, 0);  // uniform
   }
 }
 
@@ -5343,23 +5433,59 @@ hipError_t run_inflate_general(hipStream_t stream, Scratch& scratch, const u8* i
   // every val_chunk(n) of them (n <= pre_capacity).
   const u64 val_ranges = (pre_capacity + kValPerWave - 1) / kValPerWave;
   const u64 val_waves = std::max(val_ranges, std::min(pre_capacity, kValResident));
-  u32 *wg_count = nullptr, *wave_valid = nullptr;
-  u64 *wg_list = nullptr, *pre = nullptr, *cand = nullptr;
-  HZ_TRY(scratch.alloc(&wg_count, groups));
-  HZ_TRY(scratch.alloc(&wg_list, groups * kDiscCap));
-  HZ_TRY(scratch.alloc(&pre, pre_capacity));
-  HZ_TRY(scratch.alloc(&wave_valid, val_ranges));
+
+  // Buffers read by no launch after chain selection.  The roots, written from
+  // emission on, take their place.
   const u64 cand_capacity = u64(max_candidates) + 1;
-  HZ_TRY(scratch.alloc(&cand, cand_capacity));
-  // Each discovery workgroup takes per_block consecutive ranges.
-  const u64 per_block = (groups + 8191) / 8192;
+  const u64 per_block = (groups + 8191) / 8192;  // consecutive ranges of a discovery workgroup
   const u64 blocks = (groups + per_block - 1) / per_block;
-  u32* dense = nullptr;
-  u32* block_total = nullptr;
-  u64* block_base = nullptr;
-  HZ_TRY(scratch.alloc(&dense, groups));
-  HZ_TRY(scratch.alloc(&block_total, blocks));
-  HZ_TRY(scratch.alloc(&block_base, blocks));
+  const u64 rec_capacity = u64(max_blocks) + cand_capacity + 1024;
+  const u64 table_capacity = std::min<u64>(rec_capacity, len / 8192 + 1024);
+  const u64 run_capacity = cand_capacity + 1024, rt_capacity = tiles + 64 * 4096;
+  const u64 fix_group_count = tiles / kFixGroupTiles;
+  u32 *wg_count = nullptr, *wave_valid = nullptr, *dense = nullptr, *block_total = nullptr;
+  u64 *wg_list = nullptr, *pre = nullptr, *cand = nullptr, *block_base = nullptr;
+  u64 *seg_end = nullptr, *seg_size = nullptr, *hdr_d0 = nullptr;
+  u32 *seg_blocks = nullptr, *seg_next = nullptr, *seg_flags = nullptr, *exit_node = nullptr;
+  u32 *seg_rec = nullptr, *seg_last = nullptr, *region_cand = nullptr, *hdr_info = nullptr;
+  FixSummary* fix_sum = nullptr;
+  uint2* fix_entries = nullptr;
+  FixRun* fix_runs = nullptr;
+  FixTile* fix_rt = nullptr;
+  FixGroupSum* fix_groups = nullptr;
+  const auto early = [&](Scratch& s) -> hipError_t {
+    HZ_TRY(s.alloc(&wg_count, groups));
+    HZ_TRY(s.alloc(&wg_list, groups * kDiscCap));
+    HZ_TRY(s.alloc(&pre, pre_capacity));
+    HZ_TRY(s.alloc(&wave_valid, val_ranges));
+    HZ_TRY(s.alloc(&cand, cand_capacity));
+    HZ_TRY(s.alloc(&dense, groups));
+    HZ_TRY(s.alloc(&block_total, blocks));
+    HZ_TRY(s.alloc(&block_base, blocks));
+    HZ_TRY(s.alloc(&seg_end, cand_capacity));
+    HZ_TRY(s.alloc(&seg_size, cand_capacity));
+    HZ_TRY(s.alloc(&seg_blocks, cand_capacity));
+    HZ_TRY(s.alloc(&seg_next, cand_capacity));
+    HZ_TRY(s.alloc(&seg_flags, cand_capacity));
+    HZ_TRY(s.alloc(&seg_rec, cand_capacity));
+    HZ_TRY(s.alloc(&exit_node, cand_capacity));
+    HZ_TRY(s.alloc(&seg_last, cand_capacity));
+    HZ_TRY(s.alloc(&region_cand, cand_capacity));
+    HZ_TRY(s.alloc(&hdr_d0, table_capacity));
+    HZ_TRY(s.alloc(&hdr_info, table_capacity));
+    HZ_TRY(s.alloc(&fix_sum, tiles * kFixEntries));
+    HZ_TRY(s.alloc(&fix_entries, tiles));
+    HZ_TRY(s.alloc(&fix_runs, run_capacity));
+    HZ_TRY(s.alloc(&fix_rt, rt_capacity));
+    return s.alloc(&fix_groups, fix_group_count * (kFixGroupTiles / kFixGroupEvery) * 64);
+  };
+  SizingScratch sizing;
+  HZ_TRY(early(sizing));
+  u8* region = nullptr;
+  HZ_TRY(scratch.alloc(&region, std::max<u64>(sizing.total, 4 * out_total)));
+  FixedScratch early_scratch(region, sizing.total);
+  HZ_TRY(early(early_scratch));
+  u32* roots = reinterpret_cast<u32*>(region);
   HZ_LAUNCH(g_discover, dim3(u32(blocks)), dim3(kDiscThreads), 0, stream, body, len, st, wg_count,
             wg_list, dense, block_total, groups, per_block);
   HZ_TRY(hipGetLastError());
@@ -5381,30 +5507,14 @@ hipError_t run_inflate_general(hipStream_t stream, Scratch& scratch, const u8* i
   HZ_TRY(hipGetLastError());
 
   // Describe every candidate's segment.
-  u64 *seg_end = nullptr, *seg_size = nullptr;
-  u32 *seg_blocks = nullptr, *seg_next = nullptr, *seg_flags = nullptr, *exit_node = nullptr;
-  u32* seg_rec = nullptr;
-  HZ_TRY(scratch.alloc(&seg_end, cand_capacity));
-  HZ_TRY(scratch.alloc(&seg_size, cand_capacity));
-  HZ_TRY(scratch.alloc(&seg_blocks, cand_capacity));
-  HZ_TRY(scratch.alloc(&seg_next, cand_capacity));
-  HZ_TRY(scratch.alloc(&seg_flags, cand_capacity));
-  HZ_TRY(scratch.alloc(&seg_rec, cand_capacity));
-  HZ_TRY(scratch.alloc(&exit_node, cand_capacity));
   // Block records and slice groups; running out only sends a segment to the
   // serial emitter.
-  const u64 rec_capacity = u64(max_blocks) + cand_capacity + 1024;
   BlockRec* recs = nullptr;
   u64* slice_entry = nullptr;
   u32 *slice_off = nullptr, *group_link = nullptr;
   HZ_TRY(scratch.alloc(&recs, rec_capacity));
-  const u64 table_capacity = std::min<u64>(rec_capacity, len / 8192 + 1024);
   BlockTables* tables = nullptr;
-  u64* hdr_d0 = nullptr;
-  u32* hdr_info = nullptr;
   HZ_TRY(scratch.alloc(&tables, table_capacity));
-  HZ_TRY(scratch.alloc(&hdr_d0, table_capacity));
-  HZ_TRY(scratch.alloc(&hdr_info, table_capacity));
   // Grid-stride kernels over candidates, segments or units launch at most one
   // workgroup per 64 body bytes (at least 256): a small stream has few of
   // them, and idle workgroups of a 4096-wide launch cost their dispatch.
@@ -5415,9 +5525,6 @@ hipError_t run_inflate_general(hipStream_t stream, Scratch& scratch, const u8* i
   HZ_TRY(scratch.alloc(&slice_entry, group_capacity * 64));
   HZ_TRY(scratch.alloc(&slice_off, group_capacity * 64));
   HZ_TRY(scratch.alloc(&group_link, group_capacity));
-  u32 *seg_last = nullptr, *region_cand = nullptr;
-  HZ_TRY(scratch.alloc(&seg_last, cand_capacity));
-  HZ_TRY(scratch.alloc(&region_cand, cand_capacity));
   u32* fix_need = reinterpret_cast<u32*>(zeroed + 8 * zero_u64 + 4 * words);
   HZ_LAUNCH(g_describe, dim3(clamp_grid(std::min(cand_capacity, items_cap), 4096)), dim3(kDescThreads), 0, stream, body, len,
             cand, st, out_size, seg_end, seg_size, seg_blocks, seg_next, seg_flags, seg_rec, recs,
@@ -5430,37 +5537,23 @@ hipError_t run_inflate_general(hipStream_t stream, Scratch& scratch, const u8* i
 
   // Long fixed-Huffman runs deferred by describe (each launch returns at once
   // when there are none).
-  FixSummary* fix_sum = nullptr;
-  FixRun* fix_runs = nullptr;
-  FixTile* fix_rt = nullptr;
-  const u64 run_capacity = cand_capacity + 1024;
-  const u64 rt_capacity = tiles + 64 * 4096;
-  FixTask* fix_tasks = nullptr;
-  const u64 task_capacity = 4 * tiles + 4096;  // beyond it, g_fix_sum decodes the rests itself
-  HZ_TRY(scratch.alloc(&fix_sum, (tiles ? tiles : 1) * kFixEntries));
-  HZ_TRY(scratch.alloc(&fix_tasks, task_capacity));
-  HZ_TRY(scratch.alloc(&fix_runs, run_capacity));
-  HZ_TRY(scratch.alloc(&fix_rt, rt_capacity));
-  HZ_LAUNCH(g_fix_sum, dim3(clamp_grid((tiles + 7) / 8, 2048)), dim3(256), 0, stream, body, len,
-            st, fix_need, fix_sum, tiles, fix_tasks, task_capacity);
+  HZ_LAUNCH(g_fix_sum, dim3(clamp_grid(tiles, 2048)), dim3(kFixThreads), 0, stream, body, len, st,
+            fix_need, fix_sum, tiles);
   HZ_TRY(hipGetLastError());
-  HZ_LAUNCH(g_fix_rem, dim3(clamp_grid((task_capacity + 255) / 256, 2048)), dim3(256), 0, stream,
-            body, len, st, fix_tasks, task_capacity, fix_sum);
-  HZ_TRY(hipGetLastError());
-  FixGroupSum* fix_groups = nullptr;
-  const u64 fix_group_count = tiles / kFixGroupTiles;
-  HZ_TRY(scratch.alloc(&fix_groups, (fix_group_count ? fix_group_count : 1) * 64));
-  HZ_LAUNCH(g_fix_groups, dim3(clamp_grid((fix_group_count * 64 + 255) / 256, 2048)), dim3(256), 0,
-            stream, st, fix_need, fix_sum, tiles, fix_groups);
+  HZ_LAUNCH(g_fix_groups, dim3(clamp_grid(fix_group_count, 1024)), dim3(256), 0, stream, st, fix_need, fix_sum, tiles, fix_groups);
   HZ_TRY(hipGetLastError());
   HZ_LAUNCH(g_fix_walk, dim3(clamp_grid(std::min(cand_capacity, items_cap), 2048)), dim3(kWave), 0, stream, body, len, st,
             cand, fix_need, fix_sum, tiles, seg_end, seg_size, seg_blocks, seg_next, seg_flags,
             seg_rec, seg_last, region_cand, recs, rec_capacity, fix_runs, run_capacity, fix_rt,
             rt_capacity, group_link, group_capacity, out_size, fix_groups);
   HZ_TRY(hipGetLastError());
-  HZ_LAUNCH(g_fix_slices, dim3(clamp_grid((rt_capacity * kFixGroupTiles + 255) / 256, 2048)),
-            dim3(256), 0, stream, body, len, st, fix_rt, rt_capacity, fix_runs, run_capacity,
-            fix_sum, slice_entry, slice_off);
+  HZ_LAUNCH(g_fix_expand, dim3(clamp_grid(fix_group_count, 1024)), dim3(256), 0, stream, st,
+            fix_rt, rt_capacity, fix_sum, fix_entries);
+  HZ_TRY(hipGetLastError());
+  // A walk takes slots 64 at a time and uses the first of them: 61 spreads them.
+  const u32 fix_x = clamp_grid(tiles / kFixGroupTiles + 1, 61);
+  HZ_LAUNCH(g_fix_slices, dim3(fix_x, kFixGroupTiles), dim3(kFixThreads), 0, stream, body, len, st,
+            fix_rt, rt_capacity, fix_runs, run_capacity, fix_entries, slice_entry, slice_off);
   HZ_TRY(hipGetLastError());
 
   // Chain selection, then the exact walk if the fast chain declined.
@@ -5479,8 +5572,6 @@ hipError_t run_inflate_general(hipStream_t stream, Scratch& scratch, const u8* i
   u64* adler_parts = reinterpret_cast<u64*>(zeroed);
   u64* left = adler_parts + 2 * u64(3 * kAdlerSlots);
   u32* bits0 = reinterpret_cast<u32*>(left + 1);
-  u32* roots = nullptr;
-  HZ_TRY(scratch.alloc(&roots, out_total ? out_total : 1));
   u8* marks0 = zeroed + 8 * zero_u64 + 4 * words + 4 * need_words;
   const u64 out_end = out_total;  // a byte at position p is stream byte n - (out_end - p)
   // Emission by segments, then the queued units of long fixed runs.

@@ -129,6 +129,16 @@ struct FixedScratch final : Scratch {
   }
 };
 
+// Only adds up the bytes asked for; every pointer is null.
+struct SizingScratch final : Scratch {
+  u64 total = 0;
+  hipError_t alloc_bytes(void** p, u64 bytes) override {
+    *p = nullptr;
+    total += scratch_round(bytes);
+    return hipSuccess;
+  }
+};
+
 // deflate.hip: chunked encode of one stream / a batch of streams.
 // deflate_scratch_bytes: the scratch run_deflate takes for one stream.
 u64 deflate_scratch_bytes(u64 in_size, u32 chunk_bytes);

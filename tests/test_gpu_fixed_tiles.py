@@ -1,0 +1,85 @@
+"""Fixed-Huffman runs around the edges of 1 KiB tiles and groups of 64 tiles:
+runs that start and end inside a tile, at its edges, and across groups, at every
+alignment of the stream."""
+
+import zlib
+
+import numpy as np
+import pytest
+
+import workloads
+from oracle import oracle
+
+pytestmark = pytest.mark.gpu
+
+
+def _fixed(data, every=0):
+    c = zlib.compressobj(1, zlib.DEFLATED, 15, 8, zlib.Z_FIXED)
+    step = every or max(1, len(data))
+    out = b""
+    for i in range(0, len(data), step):
+        out += c.compress(data[i:i + step])
+        if every:
+            out += c.flush(zlib.Z_SYNC_FLUSH)
+    return out + c.flush()
+
+
+def _content(kind, n):
+    rng = np.random.default_rng(n + 17)
+    if kind == "text":
+        return workloads.text_like(n, rng)
+    if kind == "noise":  # 8- and 9-bit literals only
+        return rng.integers(0, 256, n, dtype=np.uint8).tobytes()
+    return workloads.runs_segment(n, rng)  # nearly every token a match of 258
+
+
+def _check(gpu, stream, raw, skew):
+    """Decodes a device tensor that starts `skew` bytes into its storage."""
+    import cuda_zlib
+    import torch
+    held = torch.from_numpy(np.frombuffer(b"\xff" * skew + stream + b"\xff" * 8, np.uint8).copy())
+    payload = held.to(gpu)[skew:skew + len(stream)]
+    out, meta = cuda_zlib.decompress_zlib_checked(payload, len(raw), gpu)
+    assert int(meta.cpu().numpy()[0]) == 0
+    assert out.cpu().numpy().tobytes() == raw
+
+
+@pytest.mark.parametrize("kind", ["text", "noise", "runs"])
+@pytest.mark.parametrize("size", [66000, 70001, 131072, 140003, 1000003])
+def test_runs_of_every_length(gpu, kind, size):
+    raw = _content(kind, size)
+    _check(gpu, _fixed(raw), raw, size % 4)
+
+
+@pytest.mark.parametrize("every", [150, 700, 1024, 1700, 66000, 120001])
+def test_runs_that_start_and_end_inside_tiles(gpu, every):
+    raw = _content("text", 300007)
+    _check(gpu, _fixed(raw, every), raw, every % 4)
+
+
+@pytest.mark.parametrize("end", [1024, 2048, 64 * 1024, 128 * 1024])
+def test_runs_that_end_at_tile_and_group_edges(gpu, end):
+    """Streams cut by a byte at a time to end just before, at and after an edge
+    of the body (whose first byte is the stream's third)."""
+    import cuda_zlib
+    data = _content("noise", 2 * end)
+    for tail in range(-2, 4):
+        n = int((end + tail) * 8 / 8.44)
+        raw = data[:n]
+        stream = _fixed(raw)
+        raw = _content("noise", 70000) + raw  # past the small route, in one run
+        _check(gpu, _fixed(raw), raw, tail & 3)
+        out = cuda_zlib.decompress_zlib(stream, n, gpu)
+        assert out.cpu().numpy().tobytes() == raw[70000:]
+
+
+@pytest.mark.parametrize("keep", [0.02, 0.3, 0.77, 0.999])
+def test_cut_runs_match_the_oracle(gpu, keep):
+    import cuda_zlib
+    raw = _content("text", 150001)
+    stream = _fixed(raw, 40000)
+    cut = stream[:int(len(stream) * keep)] + stream[-4:]
+    _, want = oracle.decompress(cut, len(raw))
+    out, meta = cuda_zlib.decompress_zlib_checked(cut, len(raw), gpu)
+    assert want and int(meta.cpu().numpy()[0]) == want
+    assert not out.any()
