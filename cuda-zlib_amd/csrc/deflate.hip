@@ -540,13 +540,9 @@ __device__ void rle_lengths_wave(TreeShared& sh) {
   u32 carry = 0;
 #pragma unroll
   for (u32 c = 0; c < 5; ++c) {
-    u32 x = cnt[c];
-    for (u32 off = 1; off < 64; off <<= 1) {
-      const u32 y = __shfl_up(x, off, 64);
-      if (lane >= off) x += y;
-    }
+    const u32 x = wave_scan_add(cnt[c]);
     u32 at_sym = carry + x - cnt[c];
-    carry += __shfl(x, 63, 64);
+    carry += u32(__builtin_amdgcn_readlane(int(x), 63));
     if (cnt[c])
       rle_run(v[c], run[c], [&](u32 sym) {
         tab.rle[at_sym++] = u16(sym);
@@ -585,11 +581,7 @@ __device__ __forceinline__ void or_bits(u32* ring, u32 pos, u64 v) {
 // prefix and writes the total.  Contains barriers: every thread must call it.
 __device__ __forceinline__ u32 block_scan(u32* scan, u32 v, u32& total) {
   const u32 lane = lane_id(), wave = threadIdx.x >> 6;
-  u32 x = v;
-  for (u32 off = 1; off < 64; off <<= 1) {
-    const u32 y = __shfl_up(x, off, 64);
-    if (lane >= off) x += y;
-  }
+  const u32 x = wave_scan_add(v);
   if (lane == 63) scan[wave] = x;
   lds_barrier();
   u32 before = 0;

@@ -228,6 +228,28 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// Inclusive prefix sum and maximum over the wave's 64 lanes (all active), by
+// DPP moves in the VALU: shifts inside the rows of 16 lanes, then the rows'
+// last lanes broadcast to the rows after.  A step is one instruction of a few
+// cycles; the shuffle it replaces (ds_bpermute) is an LDS round trip.
+template <class Op>
+__device__ __forceinline__ u32 wave_scan(u32 x, u32 identity, Op op) {
+  const int id = int(identity);
+  x = op(x, u32(__builtin_amdgcn_update_dpp(id, int(x), 0x111, 0xf, 0xf, false)));  // row_shr:1
+  x = op(x, u32(__builtin_amdgcn_update_dpp(id, int(x), 0x112, 0xf, 0xf, false)));  // row_shr:2
+  x = op(x, u32(__builtin_amdgcn_update_dpp(id, int(x), 0x114, 0xf, 0xf, false)));  // row_shr:4
+  x = op(x, u32(__builtin_amdgcn_update_dpp(id, int(x), 0x118, 0xf, 0xf, false)));  // row_shr:8
+  x = op(x, u32(__builtin_amdgcn_update_dpp(id, int(x), 0x142, 0xa, 0xf, false)));  // row_bcast:15
+  x = op(x, u32(__builtin_amdgcn_update_dpp(id, int(x), 0x143, 0xc, 0xf, false)));  // row_bcast:31
+  return x;
+}
+__device__ __forceinline__ u32 wave_scan_add(u32 x) {
+  return wave_scan(x, 0u, [](u32 a, u32 b) { return a + b; });
+}
+__device__ __forceinline__ i32 wave_scan_max(i32 x, i32 lowest) {
+  return i32(wave_scan(u32(x), u32(lowest), [](u32 a, u32 b) { return u32(max(i32(a), i32(b))); }));
+}
+
 __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
@@ -523,15 +545,7 @@ __device__ u32 huff_build_wave(HuffTable<N, P>& t, const u8* lens, u32 n, bool e
   {
     const bool used = lane >= 1 && lane <= limit && lane < 16;
     const u32 c = used ? cnt : 0u;
-    u32 wsum = c << (15 - (lane & 15)), csum = c;
-#pragma unroll
-    for (u32 o = 1; o < 16; o <<= 1) {
-      const u32 wy = __shfl_up(wsum, o, 64), cy = __shfl_up(csum, o, 64);
-      if (lane >= o) {
-        wsum += wy;
-        csum += cy;
-      }
-    }
+    const u32 wsum = wave_scan_add(c << (15 - (lane & 15))), csum = wave_scan_add(c);
     const u32 total = u32(__builtin_amdgcn_readlane(int(wsum), 15));
     const u64 lens_used = __ballot(used && cnt);
     const u64 over_limit = __ballot(lane > limit && lane < 16 && cnt);
@@ -1350,12 +1364,7 @@ __device__ inline u32 header_lengths_wave(const u32* words, Tables& tables, u32*
     const bool on = (path >> lane) & 1;
     // Lengths before each path symbol.
     const u32 r_on = on ? rep : 0u;
-    u32 incl = r_on;
-#pragma unroll
-    for (u32 o = 1; o < 64; o <<= 1) {
-      const u32 y = __shfl_up(incl, o, 64);
-      if (lane >= o) incl += y;
-    }
+    const u32 incl = wave_scan_add(r_on);
     const u32 before = i + incl - r_on;
     // The first path symbol that ends the walk, and how.
     const bool stuck = !adv;
@@ -1369,12 +1378,7 @@ __device__ inline u32 header_lengths_wave(const u32* words, Tables& tables, u32*
     const u64 valid = end < 64 ? path & ((2ull << end) - 1) : path;
     // The value a 16 repeats: that of the last other path symbol before it
     // (17 and 18 give 0), or the value carried from the earlier batches.
-    int last = (valid >> lane) & 1 && sym != 16 ? int(lane) : -1;
-#pragma unroll
-    for (u32 o = 1; o < 64; o <<= 1) {
-      const int y = __shfl_up(last, o, 64);
-      if (lane >= o && y > last) last = y;
-    }
+    const int last = wave_scan_max((valid >> lane) & 1 && sym != 16 ? int(lane) : -1, -1);
     const u32 src_sym = u32(__shfl(int(sym), last < 0 ? 0 : last, 64));
     const u32 base = last < 0 ? prev : src_sym < 16 ? src_sym : 0u;
     const u32 value = sym < 16 ? sym : sym == 16 ? base : 0u;

@@ -477,14 +477,9 @@ __device__ u64 validate_mask(const u8* body, u64 len, u64 b0, u64 pre, u8* lut, 
 }
 
 __device__ __forceinline__ u32 block_exclusive_scan(u32 v, u32* sh, u32& total) {
-  // 256-thread exclusive scan: wave shuffles, then the four wave totals.
+  // 256-thread exclusive scan: wave scans, then the four wave totals.
   const u32 t = threadIdx.x, lane = lane_id(), wave = t >> 6;
-  u32 incl = v;
-#pragma unroll
-  for (u32 off = 1; off < 64; off <<= 1) {
-    const u32 y = __shfl_up(incl, off, 64);
-    if (lane >= off) incl += y;
-  }
+  const u32 incl = wave_scan_add(v);
   if (lane == 63) sh[wave] = incl;
   __syncthreads();
   u32 before = 0;
@@ -536,12 +531,7 @@ __device__ u64 wg_exclusive_scan(const u32* in, u32 mask, u64 count, u64* out, S
     u32 mine = 0;
 #pragma unroll
     for (u32 k = 0; k < kScanPer; ++k) mine += sh.v[scan_slot(t * kScanPer + k)];
-    u32 incl = mine;
-#pragma unroll
-    for (u32 off = 1; off < 64; off <<= 1) {
-      const u32 y = __shfl_up(incl, off, 64);
-      if (lane >= off) incl += y;
-    }
+    const u32 incl = wave_scan_add(mine);
     if (lane == 63) sh.wave[wave] = incl;
     lds_barrier();
     u64 run = carry, tile_total = 0;
@@ -789,13 +779,8 @@ __global__ __launch_bounds__(256) void g_discover(const u8* body, u64 len, State
     const u32 wave_bit0 = wave * 64 * 64;  // first offset of the wave's span (range-relative)
     for (;;) {
       const u32 cnt = __popcll(m);
-      u32 incl = cnt;
-  #pragma unroll
-      for (u32 off = 1; off < 64; off <<= 1) {
-        const u32 y = __shfl_up(incl, off, 64);
-        if (lane >= off) incl += y;
-      }
-      const u32 total = __shfl(incl, 63, 64), excl = incl - cnt;
+      const u32 incl = wave_scan_add(cnt);
+      const u32 total = u32(__builtin_amdgcn_readlane(int(incl), 63)), excl = incl - cnt;
       if (!total) break;
       const u32 take = excl >= kSurvivorCap ? 0u : min(cnt, kSurvivorCap - excl);
       for (u32 k = 0; k < take; ++k) {
@@ -2013,11 +1998,7 @@ __device__ void describe_round(u64 len, u64 limit, DescShared& sh, State* st, u6
   u32 bsl = sh.count[t] - before;
   if (q != kNoEvent) bsl = at_event - before;
   else if (t + 1 < kDescThreads && sh.merge[t + 1] != kNoMerge) bsl += sh.tail[t];
-  u32 x = bsl;
-  for (u32 o = 1; o < 64; o <<= 1) {
-    const u32 y = __shfl_up(x, o, 64);
-    if (lane >= o) x += y;
-  }
+  u32 x = wave_scan_add(bsl);
   if (lane == 63) sh.wsum[wave] = x;
   const u64 bm = __ballot(t > 0 && sh.merge[t] == kNoMerge);
   const u64 em = __ballot(q != kNoEvent);
