@@ -2858,10 +2858,12 @@ __global__ __launch_bounds__(256) void g_fix_groups(const State* st, const u32* 
 }
 
 // The true entries of the tiles a walk stepped over in groups: per slot of
-// more than one tile, the entry bit (low 5 bits of x) and the run's output
-// bytes before (y) of every tile after the first, at the tile's index.  A tile
-// lies in one such step only (a run that starts in a step's last tile enters
-// that tile past its 32 entry bits: a stored block lies between).
+// more than one tile, the entry bit (low 5 bits of x), the slot (the rest) and
+// the run's output bytes before (y) of every tile after the first, at the
+// tile's index.  Steps of one walk do not share such a tile (a run that starts
+// in a step's last tile enters it past its 32 entry bits: a stored block lies
+// between), but those of two walks may (a look-alike of a candidate inside a
+// run starts a second walk over it): the slot tells whose entry was kept.
 __global__ __launch_bounds__(256) void g_fix_expand(const State* st, const FixTile* rt,
                                                     u64 rt_capacity, const FixSummary* sum,
                                                     uint2* entries) {
@@ -2882,7 +2884,7 @@ __global__ __launch_bounds__(256) void g_fix_expand(const State* st, const FixTi
         const FixSummary f = all[j - 1][e & 31u];
         off += f.bytes;
         e = f.exit - kFixTileBits;
-        if (threadIdx.x == j) mine = make_uint2(e & 31u, off);
+        if (threadIdx.x == j) mine = make_uint2((e & 31u) | (u32(i) << 5), off);
       }
       if (threadIdx.x && threadIdx.x < ft.tiles) entries[u64(ft.k) + threadIdx.x] = mine;
     }
@@ -3223,18 +3225,21 @@ __global__ __launch_bounds__(64) void g_fix_walk(
 // its slot) decodes it as g_fix_sum does and follows the slice summaries from
 // the tile's true entry: slice b - b0 of the run starts at the first token at
 // or after bit 512 b; where the run ends first, at the run's end, with nothing
-// to decode.
+// to decode.  Where another walk's entry of the tile was kept, the summaries
+// are followed from the slot's first tile.
 __global__ __launch_bounds__(kFixThreads) void g_fix_slices(const u8* body, u64 len,
                                                             const State* st, const FixTile* rt,
                                                             u64 rt_capacity, const FixRun* runs,
-                                                            u64 run_capacity, const uint2* entries,
+                                                            u64 run_capacity,
+                                                            const FixSummary* sum,
+                                                            const uint2* entries,
                                                             u64* slice_entry, u32* slice_off) {
   __shared__ FixTileShared sh;
   if (st->status || !st->fix_regions) return;
   const u64 used = min<u64>(st->fix_rt, rt_capacity);
   const u64 nruns = min<u64>(st->fix_runs, run_capacity);
   bool built = false;
-  const auto tile = [&](const FixTile& ft, u32 j) {
+  const auto tile = [&](const FixTile& ft, u64 i, u32 j) {
     const FixRun run = runs[ft.run];
     if (!run.lanes) return;
     if (!built) fix_build_lut(sh.lut);
@@ -3244,8 +3249,17 @@ __global__ __launch_bounds__(kFixThreads) void g_fix_slices(const u8* body, u64 
     u32 p = u32(ft.pos - tile0), off = ft.off;
     if (j) {
       const uint2 e = entries[k];
-      p = e.x;
-      off = e.y;
+      if (e.x >> 5 == u32(i)) {  // uniform
+        p = e.x & 31u;
+        off = e.y;
+      } else {
+        for (u32 q = 0; q < j; ++q) {
+          const FixSummary f = sum[(u64(ft.k) + q) * kFixEntries + (p & 31u)];
+          off += f.bytes;
+          p = f.exit - kFixTileBits;
+        }
+        p &= 31u;
+      }
     }
     // A run starts anywhere in a tile; every later entry is a summary's.
     const bool inside = p % kFixSliceBits >= kFixEntries;
@@ -3274,12 +3288,12 @@ __global__ __launch_bounds__(kFixThreads) void g_fix_slices(const u8* body, u64 
   // dealt over the whole grid.
   for (u64 i = blockIdx.x; i < used; i += gridDim.x) {
     const FixTile ft = rt[i];
-    if (ft.run < nruns && ft.tiles > 1 && blockIdx.y < ft.tiles) tile(ft, blockIdx.y);  // uniform
+    if (ft.run < nruns && ft.tiles > 1 && blockIdx.y < ft.tiles) tile(ft, i, blockIdx.y);  // uniform
   }
   for (u64 i = blockIdx.x + u64(gridDim.x) * blockIdx.y; i < used;
        i += u64(gridDim.x) * gridDim.y) {
     const FixTile ft = rt[i];
-    if (ft.run < nruns && ft.tiles == 1) tile(ft, 0);  // uniform
+    if (ft.run < nruns && ft.tiles == 1) tile(ft, i, 0);  // uniform
   }
 }
 
@@ -4373,6 +4387,10 @@ __global__ __launch_bounds__(kEmitThreads) __attribute__((amdgpu_waves_per_eu(4)
           // the output position `lo16` (16-byte aligned in memory), as far
           // as the stage reaches; any rest goes straight to the output.
           const u64 lo = sh.round_lo, hi = sh.round_hi;
+          if (lo < block_out || hi < lo || hi > block_out + rec.size) {  // uniform
+            error = kExtent;  // never from a consistent describe or walk
+            break;
+          }
           const u64 skew = (reinterpret_cast<uintptr_t>(out) + lo) & 15u;
           const u64 lo16 = lo - skew;
           const u64 split = min<u64>(hi, lo16 + kOutStage);
@@ -5521,7 +5539,7 @@ hipError_t run_inflate_general(hipStream_t stream, Scratch& scratch, const u8* i
   // A walk takes slots 64 at a time and uses the first of them: 61 spreads them.
   const u32 fix_x = clamp_grid(tiles / kFixGroupTiles + 1, 61);
   HZ_LAUNCH(g_fix_slices, dim3(fix_x, kFixGroupTiles), dim3(kFixThreads), 0, stream, body, len, st,
-            fix_rt, rt_capacity, fix_runs, run_capacity, fix_entries, slice_entry, slice_off);
+            fix_rt, rt_capacity, fix_runs, run_capacity, fix_sum, fix_entries, slice_entry, slice_off);
   HZ_TRY(hipGetLastError());
 
   // Chain selection, then the exact walk if the fast chain declined.

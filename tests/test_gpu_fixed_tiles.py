@@ -83,3 +83,57 @@ def test_cut_runs_match_the_oracle(gpu, keep):
     out, meta = cuda_zlib.decompress_zlib_checked(cut, len(raw), gpu)
     assert want and int(meta.cpu().numpy()[0]) == want
     assert not out.any()
+
+
+def _fixed_tokens(body, bit, count):
+    """Whether `count` fixed-code tokens decode from body bit `bit` on, a fixed block's header first."""
+    bits = int.from_bytes(body[bit // 8:bit // 8 + 8 * count], "little") >> (bit & 7)
+
+    def code(n, at):
+        return int(format((bits >> at) & ((1 << n) - 1), "0%db" % n)[::-1], 2)
+
+    if (bits >> 1) & 3 != 1:
+        return False
+    at = 3
+    for _ in range(count):
+        c7, c8 = code(7, at), code(8, at)
+        if c7 == 0:
+            return False
+        if c7 < 24 or 0xc0 <= c8 < 0xc8:
+            symbol = 256 + c7 if c7 < 24 else 280 + c8 - 0xc0
+            at += 7 if c7 < 24 else 8
+            if symbol > 285:
+                return False
+            at += 0 if symbol < 265 or symbol == 285 else (symbol - 261) // 4
+            distance = code(5, at)
+            if distance > 29:
+                return False
+            at += 5 + (0 if distance < 4 else distance // 2 - 1)
+        else:
+            at += 8 if c8 < 0xc0 else 9
+    return True
+
+
+@pytest.mark.parametrize("seed", [1, 2, 3])
+def test_second_walk_over_a_run(gpu, no_cpu_codec, seed):
+    """A stored block's payload ends in what looks like stored headers, the last of which
+    leads into the fixed run behind it: two walks cover the run's tiles."""
+    import cuda_zlib
+    text = workloads.text_like(3 << 20, np.random.default_rng(seed))
+    c = zlib.compressobj(1, zlib.DEFLATED, -15, 8, zlib.Z_FIXED)
+    run = c.compress(text) + c.flush()
+
+    def header(n):
+        return b"\0" + n.to_bytes(2, "little") + (n ^ 0xffff).to_bytes(2, "little")
+
+    skip = next(n for n in range(1000 + 7000 * seed, 65000) if _fixed_tokens(run, 8 * n, 400))
+    pad = np.random.default_rng(seed).integers(2, 256, 6000, dtype=np.uint8).tobytes()
+    payload = pad + header(5) + b"abcde" + header(skip)
+    body = header(len(payload)) + payload + run
+    data = payload + text
+    stream = b"\x78\x9c" + body + zlib.adler32(data).to_bytes(4, "big")
+    assert zlib.decompress(stream) == data
+    with no_cpu_codec:
+        out, meta = cuda_zlib.decompress_zlib_checked(stream, len(data), 0)
+    assert int(meta.cpu().numpy()[0]) == 0
+    assert out.cpu().numpy().tobytes() == data
