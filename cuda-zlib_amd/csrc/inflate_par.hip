@@ -52,6 +52,7 @@ struct State {
   u32 chain_ok;      // fast chain accepted the stream
   u64 candidates;    // dynamic candidates + bit 0 (sorted list length)
   u64 seeds;         // stored-endpoint seeds (counted for the overflow check)
+  u64 stored;        // stored-block candidates (not counted for it)
   u64 accepted;      // number of accepted segments
   u32 emit_status;
   u32 pad;
@@ -356,6 +357,29 @@ __device__ __forceinline__ bool stored_seed(const u8* body, u64 len, u64 byte) {
   for (u32 gap = 3; gap <= 10; ++gap)
     if (byte * 8 >= gap && ((before >> (17 - gap)) & 3u) == 0) possible = true;
   return possible && ((body[byte + 4 + n] >> 1) & 3u) == 1;
+}
+
+// Whether body[byte] begins a stored block as all of a chain of them but the
+// first do: BFINAL, BTYPE 0, zero padding to the byte's end, LEN and NLEN.
+__device__ __forceinline__ bool stored_header(const u8* body, u64 len, u64 byte, u64& end) {
+  if (byte > len || len - byte < 5 || body[byte] > 1) return false;
+  const u32 n = body[byte + 1] | (u32(body[byte + 2]) << 8);
+  const u32 comp = body[byte + 3] | (u32(body[byte + 4]) << 8);
+  end = byte + 5 + n;
+  return (n ^ comp) == 0xffffu && end <= len;
+}
+
+// Whether a stored block starts at `byte` and is followed by another, or is
+// the final one: candidates of their own, so that a chain of stored blocks is
+// described and copied by a workgroup each (as one segment, 32 MiB of random
+// bytes in zlib's 16 KB stored blocks took 16.3 ms, now 0.6 ms).
+// They are optional: a block that none stands for is walked by the segment
+// before it.  A header alone shows up in coded data too (9 times in 12 MB of
+// fixed codes, each a second walk of the run), two in a row practically never.
+__device__ __forceinline__ bool stored_block(const u8* body, u64 len, u64 byte) {
+  u64 end, after;
+  if (!stored_header(body, len, byte, end)) return false;
+  return (body[byte] & 1u) ? end == len : stored_header(body, len, end, after);
 }
 
 // stage_range split in two, so that a range's words can be loaded into
@@ -685,6 +709,7 @@ __global__ __launch_bounds__(256) void g_frame(const u8* in, u64 in_size, u32 fo
   st->chain_ok = 0;
   st->candidates = 0;
   st->seeds = 0;
+  st->stored = 0;
   st->accepted = 0;
   st->emit_status = 0;
   st->unresolved = 0;
@@ -704,7 +729,8 @@ __global__ __launch_bounds__(256) void g_frame(const u8* in, u64 in_size, u32 fo
 // Discovery pass 1, per 2 KiB range: prefiltered offsets in order (kind 0,
 // validated later one per lane).  A range with more than kDiscCap of them
 // validates them itself and keeps the valid ones (kind 1), or, when even those
-// overflow, leaves them to the gather pass (kind 2).  Also counts
+// overflow, leaves them to the gather pass (kind 2).  The first stored block of
+// a range that starts on a byte joins a kind 0 list as valid.  Also counts
 // stored-endpoint seeds.  Workgroups take ranges grid-stride.
 __global__ __launch_bounds__(256) void g_discover(const u8* body, u64 len, State* st,
                                                   u32* wg_count, u64* wg_list, u32* dense,
@@ -721,6 +747,7 @@ __global__ __launch_bounds__(256) void g_discover(const u8* body, u64 len, State
   __shared__ u32 scan[kDiscThreads];
   __shared__ u16 kraft3[512];
   __shared__ PreStage sg;
+  __shared__ u32 stored;  // range bit of the range's first stored block
   auto& luts = lds.luts;
   auto& surv = lds.surv;
   auto& pass = lds.pass;
@@ -735,10 +762,12 @@ __global__ __launch_bounds__(256) void g_discover(const u8* body, u64 len, State
   // This workgroup's ranges: per_block consecutive ones.
   const u64 r0 = u64(blockIdx.x) * per_block, r1 = min(groups, r0 + per_block);
   u32 entries = 0;  // listed entries of the block's ranges
+  u32 stored_listed = 0;
   if (r0 < r1) next.load(body, len, r0 * kDiscRange * 8, (r0 + 1) * kDiscRange * 8, kPreMargin);
   for (u64 wg = r0; wg < r1; ++wg) {
     next.store(sg, body);
     for (u32 i = t; i < kDiscRange * 8 / 32; i += kDiscThreads) pass[i] = 0;
+    if (!t) stored = ~0u;
     __syncthreads();
     // Words past the staged ones read as zero, as body bits past the end do.
     for (u32 i = sg.count + t; i < kPreStageWords; i += kDiscThreads) sg.words[i] = 0;
@@ -767,12 +796,16 @@ __global__ __launch_bounds__(256) void g_discover(const u8* body, u64 len, State
       if (bits_left < 64) m &= (1ull << bits_left) - 1;
       m &= allowed;
     }
-    // Stored-endpoint seeds: LEN/NLEN complement in the staged bytes first.
+    // Stored-endpoint seeds and stored blocks: LEN/NLEN complement in the
+    // staged bytes first.
   #pragma unroll
-    for (u32 j = 0; j < kDiscBytesPerThread; ++j) {
-      const u32 x = u32(funnel(w0, w1, 8 * j));
-      if (((x ^ (x >> 16)) & 0xffffu) == 0xffffu && b0 + j < len && stored_seed(body, len, b0 + j))
-        ++seeds;
+    for (u32 j = 0; j <= kDiscBytesPerThread; ++j) {
+      const u32 x = j < kDiscBytesPerThread ? u32(funnel(w0, w1, 8 * j)) : u32(w1);
+      if (((x ^ (x >> 16)) & 0xffffu) == 0xffffu && b0 + j < len) {
+        if (j < kDiscBytesPerThread && stored_seed(body, len, b0 + j)) ++seeds;
+        if (j && ((allowed >> (8 * (j ? j - 1 : 0))) & 1) && stored_block(body, len, b0 + j - 1))
+          atomicMin(&stored, 64 * t + 8 * (j - 1));
+      }
     }
     // Complete code-length code (Kraft sum of the HCLEN lengths == 128) for
     // the survivors, compacted per wave so that every lane checks one.
@@ -811,13 +844,15 @@ __global__ __launch_bounds__(256) void g_discover(const u8* body, u64 len, State
     __syncthreads();
     u64 mask = u64(pass[2 * t]) | (u64(pass[2 * t + 1]) << 32);
     const u64 flag = first;  // the first block is always a candidate
-    mask |= first;
-    u64 valid_flag = flag;
+    const u64 stored_flag = stored >> 6 == t ? 1ull << (stored & 63u) : 0ull;
+    mask |= first | stored_flag;
+    u64 valid_flag = flag | stored_flag;
     u32 total;
     u32 base = block_exclusive_scan(__popcll(mask), scan, total);
     u32 kind = 0;
     if (total > kDiscCap) {
-      mask = validate_mask(body, len, b0, mask & ~flag, &luts[0][threadIdx.x], kDiscThreads) | flag;
+      mask = validate_mask(body, len, b0, mask & ~valid_flag, &luts[0][threadIdx.x], kDiscThreads) |
+             flag;
       valid_flag = mask;
       base = block_exclusive_scan(__popcll(mask), scan, total);
       kind = total > kDiscCap ? 2u : 1u;
@@ -828,6 +863,7 @@ __global__ __launch_bounds__(256) void g_discover(const u8* body, u64 len, State
         dense[atomicAdd(reinterpret_cast<unsigned long long*>(&st->dense_count), 1ull)] = u32(wg);
     }
     entries += total;
+    if (!kind && stored_flag) ++stored_listed;
     if (kind < 2) {
       while (mask) {
         const u32 k = __builtin_ctzll(mask);
@@ -839,6 +875,8 @@ __global__ __launch_bounds__(256) void g_discover(const u8* body, u64 len, State
   }
   if (!t) block_total[blockIdx.x] = entries;
   if (seeds) atomicAdd(reinterpret_cast<unsigned long long*>(&st->seeds), seeds);
+  if (stored_listed)
+    atomicAdd(reinterpret_cast<unsigned long long*>(&st->stored), stored_listed);
 }
 
 // Offset in the dense array of range wg's list: its block's base plus the
@@ -1345,7 +1383,7 @@ __global__ __launch_bounds__(256) void g_valid_scatter(State* st, const u64* pre
     for (u32 w = 0; w < kDiscThreads / 64; ++w) total += wave_count[w];
     st->candidates = total;
     st->tables_used = total;  // table slots 0 .. total-1 belong to the candidates
-    if (total + st->seeds > max_candidates) st->status = kCandidateOverflow;
+    if (total - st->stored + st->seeds > max_candidates) st->status = kCandidateOverflow;
   }
 }
 
@@ -5422,7 +5460,8 @@ hipError_t run_inflate_general(hipStream_t stream, Scratch& scratch, const u8* i
 
   // Buffers read by no launch after chain selection.  The roots, written from
   // emission on, take their place.
-  const u64 cand_capacity = u64(max_candidates) + 1;
+  // The counted candidates and bit 0, and a stored block per range.
+  const u64 cand_capacity = u64(max_candidates) + 1 + groups;
   const u64 per_block = (groups + 8191) / 8192;  // consecutive ranges of a discovery workgroup
   const u64 blocks = (groups + per_block - 1) / per_block;
   const u64 rec_capacity = u64(max_blocks) + cand_capacity + 1024;
