@@ -66,3 +66,17 @@ def test_broken_chain(gpu, cut):
         got, status, _ = capi_decompress(stream, len(data))
         want, want_status = oracle.decompress(stream, len(data))
         assert (status, got) == (want_status, want)
+
+
+@pytest.mark.parametrize("tail", [120, 300, 520, 640, 700, 1000])
+@pytest.mark.parametrize("size", [30 * KIB, 900 * KIB])
+def test_last_header_near_the_end(gpu, size, tail):
+    """A small last dynamic block: its header ends close to the body's end."""
+    data = workloads.text_like(size, np.random.default_rng(size))
+    end = np.random.default_rng(tail).choice(np.frombuffer(b"etaoin shrdlu,.XQ", np.uint8),
+                                             tail).tobytes()
+    c = zlib.compressobj(9, zlib.DEFLATED, 15, 9, zlib.Z_HUFFMAN_ONLY)
+    stream = c.compress(data) + c.flush(zlib.Z_BLOCK) + c.compress(end) + c.flush()
+    got, status, _ = capi_decompress(stream, size + tail)
+    assert status == 0
+    assert got == data + end
