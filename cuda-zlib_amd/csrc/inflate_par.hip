@@ -32,6 +32,7 @@
 #include <algorithm>
 
 #include "deflate_common.h"
+#include "resolve_common.h"
 #include "kernels.h"
 
 namespace hz {
@@ -3738,18 +3739,13 @@ __device__ __forceinline__ void bit_set(u32* bits, u64 i) {
 
 // Copies one output byte from `src` to `dst` inside a segment starting at
 // `seg`; sources outside the segment or still unresolved make the byte
-// unresolved.  Returns true when the byte was queued.
+// unresolved, rooted at its source.  Returns true when the byte was queued.
 // Written bytes are added to Adler-32 sums S (s) and W (w), a byte at output
 // position p weighing end - p.
 __device__ __forceinline__ bool copy_byte(u8* out, u32* roots, u32* unres, u64 seg, u64 dst,
                                           u64 src, u64& s, u64& w, u64 end) {
-  if (src < seg) {
+  if (src < seg || bit_get(unres, src)) {
     roots[dst] = u32(src);
-    bit_set(unres, dst);
-    return true;
-  }
-  if (bit_get(unres, src)) {
-    roots[dst] = roots[src];
     bit_set(unres, dst);
     return true;
   }
@@ -4098,6 +4094,13 @@ __device__ __forceinline__ void roots_fill(u32* roots, u64 dst, u32 n, u32 root,
   for (; j < n; ++j) roots[dst + j] = root + j * step;
 }
 
+// The roots of a run (see run_roots); returns the last byte's.
+__device__ __forceinline__ u32 run_roots_fill(u32* roots, u64 dst, u32 n, u32 root) {
+  return run_roots(dst, n, root, [&](u64 first, u32 count, u32 r) {
+    roots_fill(roots, first, count, r, 0);
+  });
+}
+
 // out[dst + j] = out[src0 + j] for j < length where src0 + distance = dst:
 // an overlapping copy repeats the first `distance` bytes, so every byte is
 // read from [src0, dst), never from this copy's own stores.
@@ -4147,27 +4150,26 @@ __device__ __forceinline__ void emit_match(const Sink& out, u64 dst0, u64 dst, u
   const u32 at = u32(dst - dst0);
   const bool extend = kDefer && distance == 1 && (at == 0 || (lead && at == lead && tail_at == lead));
   if (kDefer && !extend && lead && src0 < dst0 + lead && src0 + length > dst0) {
-    roots_fill(roots, dst0, lead, u32(dst0 - 1), 0);
+    const u32 last = run_roots_fill(roots, dst0, lead, u32(dst0 - 1));
     bits_set_range(unres, dst0, lead);
     nunres += lead;
-    if (tail_at == lead) tail_root = u32(dst0 - 1);
+    if (tail_at == lead) tail_root = last;
     lead = 0;
   }
   if (extend) {
     lead = at + length;  // the leading run, begun or extended
     tail_root = kNone;   // not read while the tail is the leading run
   } else if (distance == 1) {
-    // A run of the byte before: one root for the whole run when that byte
-    // precedes the slice or ends an unresolved match, else resolved.
+    // A run of the byte before: unresolved, rooted at that byte or at its
+    // root, when it precedes the slice or ends an unresolved match, else
+    // resolved.
     const u64 p = dst - 1;
     const bool before = p < dst0;
     if (before || (at == tail_at && tail_root != kNone)) {
-      const u32 root = before ? u32(p) : tail_root;
-      roots_fill(roots, dst, length, root, 0);
+      tail_root = run_roots_fill(roots, dst, length, before ? u32(p) : tail_root);
       bits_set_range(unres, dst, length);
       out.zero(dst, length);
       nunres += length;
-      tail_root = root;
     } else {
       out.fill(dst, length, out.get(p));
       tail_root = kNone;
@@ -4562,7 +4564,7 @@ __global__ __launch_bounds__(kEmitThreads) __attribute__((amdgpu_waves_per_eu(4)
                 sums.w += sink.acc.w;
               } else {
                 const u32 root = before >> 32 == kLastRoot >> 32 ? u32(before) : u32(dst0 - 1);
-                roots_fill(roots, dst0, lead, root, 0);
+                run_roots_fill(roots, dst0, lead, root);
                 bits_set_range(unres, dst0, lead);
                 mark_groups(marks, dst0, lead);
                 unres_total += lead;
@@ -4854,13 +4856,12 @@ __global__ __launch_bounds__(256) void g_batch_wide_finish(const BatchFile* file
 // about every 33 KiB, so short stripes leave more).
 constexpr u32 kStripeThreads = 1024;
 constexpr u32 kStripeTile = 4 * kStripeThreads;  // bytes a step resolves, four per thread
-constexpr u32 kStripeWindow = 32768;             // the longest back-reference
+constexpr u32 kStripeWindow = kMaxBack;          // every root lies in the ring or before the stripe
 constexpr u32 kStripeRing = kStripeWindow + kStripeTile;
 constexpr u32 kStripes = 256;                    // a workgroup per CU
 constexpr u64 kStripeMin = 65536;                // output bytes below which a stripe is not cut
 // A ring entry: a byte (0 .. 255), or one of
 constexpr u32 kRingPending = 0x2000u;  // | tile offset of the byte it copies, in the same tile
-constexpr u32 kRingFar = 0x4000u;      // unresolved, its chain leaves the ring and the window before
 constexpr u32 kRingBefore = 0x8000u;   // | offset in the 32 KiB before the stripe it copies from
 static_assert(kStripeTile <= 0x2000u && kStripeTile == 2u << kResolveGroupShift,
               "tile offsets fit their tag; a tile is two mark groups");
@@ -4921,9 +4922,9 @@ constexpr u64 kStripeSparse = 64;
 // pointer jumping over roots inside the tile, all in LDS; a root before the
 // stripe stays one, tagged in the ring, and passes through every copy of it.
 // Only bytes whose chain ends before the stripe stay unresolved, with that end
-// as their root, and those whose chain meets a root more than 32 KiB back (a
-// run's), which keep the root they had.  The barriers of a tile order LDS only, so that the next tile's
-// loads stay in flight over them.
+// as their root (no root lies further back than the ring holds).  The barriers
+// of a tile order LDS only, so that the next tile's loads stay in flight over
+// them.
 // Bits, marks and roots are updated in place; the bytes left are counted in
 // *left_count.  With `parts`, every byte resolved is added to the Adler-32
 // pairs (a byte at position p weighs out_end - p).
@@ -4991,12 +4992,11 @@ g_resolve_stripes(State* st, u8* out, u32* roots, u32* bits, u8* marks, u64 out_
     for (u32 j = 0; j < 4; ++j) {
       const u32 x = r[j], d = tile0 - x;  // bytes from the root to the tile (wraps inside it)
       const bool unres = (nib >> j) & 1u, inside = x >= start32, tile = x >= tile0;
-      const bool near = inside && !tile && d <= kStripeWindow;
+      const bool near = inside && !tile;
       const u32 slot = near ? slot0 - d + (slot0 >= d ? 0u : kStripeRing) : 0u;
       const u32 ring = sh.ring[slot];
       const u32 other = tile ? kRingPending | (x - tile0)
-                        : !inside && start32 - x <= kStripeWindow
-                            ? kRingBefore | (x + kStripeWindow - start32) : kRingFar;
+                             : kRingBefore | ((x + kStripeWindow - start32) & (kRingBefore - 1u));
       e[j] = unres ? (near ? ring : other) : (bytes >> (8 * j)) & 255u;
       const bool held = (have >> (((d - 1) / kStripeTile) & 31u)) & 1u;
       direct |= u32(unres && near && !held) << j;
@@ -5040,7 +5040,7 @@ g_resolve_stripes(State* st, u8* out, u32* roots, u32* bits, u8* marks, u64 out_
 #pragma unroll
       for (u32 j = 0; j < 4; ++j) {
         if (e[j] & kRingBefore) r[j] = start32 - kStripeWindow + (e[j] & (kRingBefore - 1u));
-        if (e[j] >= kRingFar) rem |= 1u << j;
+        if (e[j] & kRingBefore) rem |= 1u << j;
         else v |= e[j] << (8 * j);
         const u32 x = ((nib & ~rem) >> j) & 1u ? e[j] : 0u;
         cs += x;
@@ -5078,21 +5078,6 @@ g_resolve_stripes(State* st, u8* out, u32* roots, u32* bits, u8* marks, u64 out_
     have = step < 32 ? ((have << 1 | 1u) << (step - 1)) & ((1u << (kRingTiles - 1)) - 1u) : 0u;
     ti = ti2;
     cur = nxt;
-  }
-  if (gridDim.x == 1 && __syncthreads_or(kept)) {
-    // The only stripe: far bytes, followed to a resolved one (no bit changes
-    // any more, and every store before is visible past the barrier).
-    for (u64 p = 8 * u64(t); p < end; p += 8 * kStripeThreads)
-      for (u32 m = bit_bytes[p >> 3]; m; m &= m - 1) {
-        const u64 u = p + u32(__builtin_ctz(m));
-        u32 x = roots[u];
-        while ((bit_bytes[x >> 3] >> (x & 7)) & 1u) x = roots[x];
-        const u32 v = out[x];
-        out[u] = u8(v);
-        as += v;
-        aw += (out_end - u) * v;
-        if (aw >> 60) aw %= kAdlerMod;
-      }
   }
   for (u32 off = 32; off; off >>= 1) kept += __shfl_down(kept, off, 64);
   if (!lane && kept) atomicAdd(reinterpret_cast<unsigned long long*>(left_count), u64(kept));
@@ -5179,8 +5164,8 @@ __device__ __forceinline__ u32 rest_end(const u32* bits, const u32* roots, u32 x
 }
 
 // The other bytes g_resolve_stripes left: their roots lie in the 32 KiB before
-// their stripe (final by now), or elsewhere (a run's, or with the stripes
-// skipped) and are followed.  A workgroup sweeps kRestBytes of a stripe: with
+// their stripe (final by now), or elsewhere (with the stripes skipped) and are
+// followed.  A workgroup sweeps kRestBytes of a stripe: with
 // few bytes left there it lists them and takes one a thread, else four
 // consecutive positions a thread.
 constexpr u32 kXcds = 8;  // MI355X: 8 accelerator complex dies of 32 CUs

@@ -43,6 +43,21 @@ def test_resolved_output(gpu, kind, size):
     assert out.cpu().numpy().tobytes() == raw
 
 
+@pytest.mark.parametrize("run", [32766, 32768, 40000, 70001])
+@pytest.mark.parametrize("size", [40000, STRIPE + 5, 9 * STRIPE + 1, 20 * STRIPE + 4093])
+def test_long_unresolved_runs(gpu, run, size):
+    """Runs longer than a back-reference whose first byte is copied, then short
+    periods copied from the run: chains of many links inside a stripe."""
+    import cuda_zlib
+    head = np.random.default_rng(run).integers(1, 7, 3000, dtype=np.uint8).tobytes()
+    unit = b"marker\0\1" + head + b"marker" + b"\0" * run + b"\0\0\0\7" * 9000
+    raw = (unit * (size // len(unit) + 1))[:size]
+    for level in (1, 6):
+        out, meta = cuda_zlib.decompress_zlib_checked(zlib.compress(raw, level), size, gpu)
+        assert int(meta.cpu().numpy()[0]) == 0
+        assert out.cpu().numpy().tobytes() == raw
+
+
 @pytest.mark.parametrize("skew", [1, 2, 3])
 def test_resolved_output_unaligned(gpu, skew):
     """An output that starts between dwords; the bytes around it stay as they were."""
