@@ -4081,24 +4081,22 @@ struct RoundBytes {
   __device__ __forceinline__ void zero(u64, u32) const {}
 };
 
-// roots[dst + j] = root + j * step for j < n, four roots a store where the
-// positions are 16-byte aligned (a run's positions are its own: no other
+// The roots of unresolved bytes (see root_range), four a store where the
+// positions are 16-byte aligned (a match's positions are its own: no other
 // thread writes them).
-__device__ __forceinline__ void roots_fill(u32* roots, u64 dst, u32 n, u32 root, u32 step) {
-  u32 j = 0;
-  for (; j < n && ((dst + j) & 3u); ++j) roots[dst + j] = root + j * step;
-  for (; j + 4 <= n; j += 4) {
-    const u32 r = root + j * step;
-    *reinterpret_cast<uint4*>(roots + dst + j) = make_uint4(r, r + step, r + 2 * step, r + 3 * step);
-  }
-  for (; j < n; ++j) roots[dst + j] = root + j * step;
-}
-
-// The roots of a run (see run_roots); returns the last byte's.
-__device__ __forceinline__ u32 run_roots_fill(u32* roots, u64 dst, u32 n, u32 root) {
-  return run_roots(dst, n, root, [&](u64 first, u32 count, u32 r) {
-    roots_fill(roots, first, count, r, 0);
-  });
+__device__ __forceinline__ u32 store_roots(u32* roots, u64 dst, u32 n, u32 root, bool run) {
+  roots += dst;
+  const u32 lead = u32(0 - dst) & 3u, mask = run ? 0u : ~0u;
+  return root_range(dst, n, root, run, [&](u32 count, u32 r) {
+    u32 j = 0;
+    for (; j < count && j < lead; ++j) roots[j] = r + (j & mask);
+    for (; j + 4 <= count; j += 4) {
+      const u32 q = r + (j & mask);
+      *reinterpret_cast<uint4*>(roots + j) =
+          make_uint4(q, q + (1 & mask), q + (2 & mask), q + (3 & mask));
+    }
+    for (; j < count; ++j) roots[j] = r + (j & mask);
+  }, [&](u32 j, u32 r) { roots[j] = r; });
 }
 
 // out[dst + j] = out[src0 + j] for j < length where src0 + distance = dst:
@@ -4136,8 +4134,9 @@ __device__ __forceinline__ void copy_periodic(const Sink& out, u64 dst, u64 src0
 // dst0 (and, once the slice has an unresolved byte, every byte it copies from
 // its own output) are marked unresolved with their root; the rest are copied.  `nunres` counts the slice's
 // unresolved bytes so far.  tail_at / tail_root: the slice offset just past
-// the last match handled, and the root of that match's last byte (kNone when
-// it is resolved): the byte before a match is that byte or a literal.
+// the last match handled, and the root of that match's last byte (kNoRoot when
+// it is resolved; see handed_root): the byte before a match is that byte or a
+// literal.
 // With kDefer, a run of the byte before the slice at the slice's start (its
 // leading run, `lead` bytes) is left unwritten and unmarked: once the round
 // is decoded, the workgroup learns that byte's value or root from the slice
@@ -4150,7 +4149,7 @@ __device__ __forceinline__ void emit_match(const Sink& out, u64 dst0, u64 dst, u
   const u32 at = u32(dst - dst0);
   const bool extend = kDefer && distance == 1 && (at == 0 || (lead && at == lead && tail_at == lead));
   if (kDefer && !extend && lead && src0 < dst0 + lead && src0 + length > dst0) {
-    const u32 last = run_roots_fill(roots, dst0, lead, u32(dst0 - 1));
+    const u32 last = store_roots(roots, dst0, lead, u32(dst0 - 1), true);
     bits_set_range(unres, dst0, lead);
     nunres += lead;
     if (tail_at == lead) tail_root = last;
@@ -4158,40 +4157,31 @@ __device__ __forceinline__ void emit_match(const Sink& out, u64 dst0, u64 dst, u
   }
   if (extend) {
     lead = at + length;  // the leading run, begun or extended
-    tail_root = kNone;   // not read while the tail is the leading run
-  } else if (distance == 1) {
-    // A run of the byte before: unresolved, rooted at that byte or at its
-    // root, when it precedes the slice or ends an unresolved match, else
-    // resolved.
-    const u64 p = dst - 1;
-    const bool before = p < dst0;
-    if (before || (at == tail_at && tail_root != kNone)) {
-      tail_root = run_roots_fill(roots, dst, length, before ? u32(p) : tail_root);
+    tail_root = kNoRoot;  // not read while the tail is the leading run
+  } else {
+    // A run of the byte before is unresolved, rooted at that byte or at its
+    // root, when it precedes the slice or ends an unresolved match.  Another
+    // copy is unresolved as a whole, every byte rooted at its source, when its
+    // source starts before the slice or the slice has an unresolved byte.  Of a
+    // source in the slice's own output it is not checked whether that is
+    // resolved (a load of the bitmap or of the source's root would wait for
+    // every store the wave has pending); a resolved source only costs
+    // resolution one link.  (With the roots and bits of copies across the
+    // slice's start set byte by byte, an atomic each, 4 KiB of text took 276 us
+    // to decode, now 226, and 609 KB of runs at level 1 6.0 ms, now 2.0.)
+    const bool run = distance == 1, before = src0 < dst0;
+    const bool unresolved = before || (run ? at == tail_at && tail_root != kNoRoot : nunres != 0);
+    if (unresolved) {
+      tail_root = store_roots(roots, dst, length, run && !before ? tail_root : u32(src0), run);
       bits_set_range(unres, dst, length);
       out.zero(dst, length);
       nunres += length;
     } else {
-      out.fill(dst, length, out.get(p));
-      tail_root = kNone;
+      // Every source is this slice's own resolved output.
+      if (run) out.fill(dst, length, out.get(src0));
+      else copy_periodic(out, dst, src0, distance, length);
+      tail_root = kNoRoot;
     }
-  } else if (!nunres && src0 >= dst0) {
-    // Every source is this slice's own resolved output.
-    copy_periodic(out, dst, src0, distance, length);
-    tail_root = kNone;
-  } else {
-    // The source starts before the slice, or the slice has an unresolved byte:
-    // every byte is rooted at its source.  Of a source in the slice's own
-    // output it is not checked whether that is resolved (a load of the bitmap
-    // or of the source's root would wait for every store the wave has
-    // pending); a resolved source only costs resolution one link.  (With the
-    // roots and bits of copies across the slice's start set byte by byte, an
-    // atomic each, 4 KiB of text took 276 us to decode, now 226, and 609 KB of
-    // runs at level 1 6.0 ms, now 2.0.)
-    roots_fill(roots, dst, length, u32(src0), 1);
-    bits_set_range(unres, dst, length);
-    out.zero(dst, length);
-    nunres += length;
-    tail_root = u32(src0) + length - 1;
   }
   tail_at = at + length;
 }
@@ -4276,7 +4266,7 @@ __device__ u32 emit_slice(Shared& sh, u32 blim, u32 entry, u32 stop, u64 dst0, u
   u64 dst = dst0;
   u32 nunres = 0, err = 0;  // unresolved bytes of this slice
   MatchQueue q;
-  u32 tail_at = 0, tail_root = kNone;  // see emit_match
+  u32 tail_at = 0, tail_root = kNoRoot;  // see emit_match
   lead = 0;
   bool live = true;
   for (;;) {
@@ -4339,7 +4329,7 @@ __device__ u32 emit_slice(Shared& sh, u32 blim, u32 entry, u32 stop, u64 dst0, u
   if (kDefer) {
     const u32 n = u32(dst - dst0);
     if (!n || lead == n) last = kLastInherit;
-    else if (tail_at == n && tail_root != kNone) last = kLastRoot | tail_root;
+    else if (tail_at == n && tail_root != kNoRoot) last = kLastRoot | tail_root;
     else last = kLastValue | out.get(dst - 1);
   }
   return err;
@@ -4564,7 +4554,7 @@ __global__ __launch_bounds__(kEmitThreads) __attribute__((amdgpu_waves_per_eu(4)
                 sums.w += sink.acc.w;
               } else {
                 const u32 root = before >> 32 == kLastRoot >> 32 ? u32(before) : u32(dst0 - 1);
-                run_roots_fill(roots, dst0, lead, root);
+                store_roots(roots, dst0, lead, root, true);
                 bits_set_range(unres, dst0, lead);
                 mark_groups(marks, dst0, lead);
                 unres_total += lead;
@@ -4855,16 +4845,14 @@ __global__ __launch_bounds__(256) void g_batch_wide_finish(const BatchFile* file
 // survives a tile's walk past the stripe's start with a share that halves
 // about every 33 KiB, so short stripes leave more).
 constexpr u32 kStripeThreads = 1024;
-constexpr u32 kStripeTile = 4 * kStripeThreads;  // bytes a step resolves, four per thread
-constexpr u32 kStripeWindow = kMaxBack;          // every root lies in the ring or before the stripe
+constexpr u32 kStripeWindow = kMaxBack;  // every root lies in the ring or before the stripe
 constexpr u32 kStripeRing = kStripeWindow + kStripeTile;
-constexpr u32 kStripes = 256;                    // a workgroup per CU
-constexpr u64 kStripeMin = 65536;                // output bytes below which a stripe is not cut
 // A ring entry: a byte (0 .. 255), or one of
 constexpr u32 kRingPending = 0x2000u;  // | tile offset of the byte it copies, in the same tile
 constexpr u32 kRingBefore = 0x8000u;   // | offset in the 32 KiB before the stripe it copies from
-static_assert(kStripeTile <= 0x2000u && kStripeTile == 2u << kResolveGroupShift,
-              "tile offsets fit their tag; a tile is two mark groups");
+static_assert(kStripeTile <= 0x2000u && kStripeTile == 2u << kResolveGroupShift &&
+                  kStripeTile == 4 * kStripeThreads,
+              "tile offsets fit their tag; a tile is two mark groups, four bytes per thread");
 
 struct StripeShared {
   __align__(16) u16 ring[kStripeRing];
@@ -4898,7 +4886,8 @@ __device__ __forceinline__ void resolve_add_parts(u64* parts, u64 as, u64 aw, u6
 struct StripeLoad {
   u32 word, w0, w1;
   uint4 roots;
-  // words: the output's aligned dwords, of which dword `last` is the last one.
+  // p: offset in the stripe, whose roots and bits these are.  words: the
+  // aligned dwords from its start on, of which dword `last` is the output's last.
   __device__ __forceinline__ void load(const u32* words, u32 skew, u32 last, const u32* root,
                                        const u32* bits, u32 p) {
     const u32 q = (p + skew) >> 2;  // p is a multiple of 4
@@ -4940,13 +4929,19 @@ g_resolve_stripes(State* st, u8* out, u32* roots, u32* bits, u8* marks, u64 out_
   }
   if (!st->unresolved) return;
   constexpr u32 kRingTiles = kStripeRing / kStripeTile;
+  // Everything from here on counts from the stripe's start.
   const u64 start = u64(blockIdx.x) * stripe_bytes;
-  const u64 end = min(start + stripe_bytes, out_end);
-  const u32 tiles = u32((end - start + kStripeTile - 1) / kStripeTile);
+  const u32 size = stripe_size(start, stripe_bytes, out_end);
+  const u64 weight = out_end - start;  // of the stripe's first byte
+  out += start;
+  roots += start;
+  bits += start >> 5;
+  marks += start >> kResolveGroupShift;
+  const u32 tiles = (size + kStripeTile - 1) / kStripeTile;
   const u32 skew = u32(reinterpret_cast<uintptr_t>(out) & 3u);
   const u32* words = reinterpret_cast<const u32*>(out - skew);
-  const u32 last = u32((out_end - 1 + skew) >> 2);
-  const u32 groups = u32((out_end + (1u << kResolveGroupShift) - 1) >> kResolveGroupShift);
+  const u32 last = u32(min<u64>((weight - 1 + skew) >> 2, 0xffffffffu));
+  const u32 groups = (size + (1u << kResolveGroupShift) - 1) >> kResolveGroupShift;
   u8* bit_bytes = reinterpret_cast<u8*>(bits);
   if (t < 4) sh.left[t >> 1][t & 1] = 0;
   __syncthreads();
@@ -4955,8 +4950,8 @@ g_resolve_stripes(State* st, u8* out, u32* roots, u32* bits, u8* marks, u64 out_
   u32 tb = 0;
   u64 marked = 0;
   const auto load_marks = [&]() {
-    const u32 mg = u32(start >> kResolveGroupShift) + 2 * tb + lane;
-    marked = __ballot(mg < groups && 2 * tb + lane < 2 * tiles && marks[mg]);
+    const u32 mg = 2 * tb + lane;
+    marked = __ballot(mg < groups && marks[mg]);
   };
   const auto next_tile = [&]() -> u32 {
     while (!marked) {
@@ -4969,8 +4964,8 @@ g_resolve_stripes(State* st, u8* out, u32* roots, u32* bits, u8* marks, u64 out_
     return tb + b;
   };
   const auto load_tile = [&](StripeLoad& l, u32 tile) {  // any tile of the stripe
-    const u32 p = u32(start) + tile * kStripeTile + 4 * t;
-    l.load(words, skew, last, roots, bits, min(p, u32(end - 1) & ~3u));
+    const u32 p = tile * kStripeTile + 4 * t;
+    l.load(words, skew, last, roots, bits, min(p, (size - 1) & ~3u));
   };
   load_marks();
   u32 ti = next_tile();
@@ -4981,22 +4976,22 @@ g_resolve_stripes(State* st, u8* out, u32* roots, u32* bits, u8* marks, u64 out_
   while (ti != kNone) {  // uniform
     const u32 ti2 = next_tile();
     load_tile(nxt, ti2 != kNone ? ti2 : ti);
-    // Positions in 32 bits, as the roots are.
-    const u32 start32 = u32(start), tile0 = start32 + ti * kStripeTile, p = tile0 + 4 * t;
+    const u32 tile0 = ti * kStripeTile, p = tile0 + 4 * t;
     const u32 slot0 = (ti % kRingTiles) * kStripeTile;
-    u32 nib = p < u32(end) ? (cur.word >> (p & 31u)) & 15u : 0u;
+    u32 nib = p < size ? (cur.word >> (p & 31u)) & 15u : 0u;
     const u32 bytes = __builtin_amdgcn_alignbyte(cur.w1, cur.w0, skew);
     u32 e[4], r[4] = {cur.roots.x, cur.roots.y, cur.roots.z, cur.roots.w};
     u32 direct = 0;  // bytes whose root's tile is not in the ring
 #pragma unroll
     for (u32 j = 0; j < 4; ++j) {
-      const u32 x = r[j], d = tile0 - x;  // bytes from the root to the tile (wraps inside it)
-      const bool unres = (nib >> j) & 1u, inside = x >= start32, tile = x >= tile0;
+      const u32 x = stripe_offset(start, r[j]);
+      const u32 d = tile0 - x;  // bytes from the root to the tile (wraps inside it)
+      const bool unres = (nib >> j) & 1u, inside = !stripe_before(x), tile = inside && x >= tile0;
       const bool near = inside && !tile;
       const u32 slot = near ? slot0 - d + (slot0 >= d ? 0u : kStripeRing) : 0u;
       const u32 ring = sh.ring[slot];
       const u32 other = tile ? kRingPending | (x - tile0)
-                             : kRingBefore | ((x + kStripeWindow - start32) & (kRingBefore - 1u));
+                             : kRingBefore | ((x + kStripeWindow) & (kRingBefore - 1u));
       e[j] = unres ? (near ? ring : other) : (bytes >> (8 * j)) & 255u;
       const bool held = (have >> (((d - 1) / kStripeTile) & 31u)) & 1u;
       direct |= u32(unres && near && !held) << j;
@@ -5004,7 +4999,7 @@ g_resolve_stripes(State* st, u8* out, u32* roots, u32* bits, u8* marks, u64 out_
     if (direct) {
       u32 v[4];
 #pragma unroll
-      for (u32 j = 0; j < 4; ++j) v[j] = out[(direct >> j) & 1u ? r[j] : tile0];
+      for (u32 j = 0; j < 4; ++j) v[j] = out[(direct >> j) & 1u ? stripe_offset(start, r[j]) : tile0];
 #pragma unroll
       for (u32 j = 0; j < 4; ++j) {
         e[j] = (direct >> j) & 1u ? v[j] : e[j];
@@ -5039,7 +5034,7 @@ g_resolve_stripes(State* st, u8* out, u32* roots, u32* bits, u8* marks, u64 out_
       u32 rem = 0, v = 0, cs = 0, cl = 0;
 #pragma unroll
       for (u32 j = 0; j < 4; ++j) {
-        if (e[j] & kRingBefore) r[j] = start32 - kStripeWindow + (e[j] & (kRingBefore - 1u));
+        if (e[j] & kRingBefore) r[j] = u32(start) - kStripeWindow + (e[j] & (kRingBefore - 1u));
         if (e[j] & kRingBefore) rem |= 1u << j;
         else v |= e[j] << (8 * j);
         const u32 x = ((nib & ~rem) >> j) & 1u ? e[j] : 0u;
@@ -5047,9 +5042,9 @@ g_resolve_stripes(State* st, u8* out, u32* roots, u32* bits, u8* marks, u64 out_
         cl += j * x;
       }
       as += cs;
-      aw += (out_end - p) * cs - cl;
+      aw += (weight - p) * cs - cl;
       if (aw >> 60) aw %= kAdlerMod;
-      if (!skew && p + 4 <= u32(end)) {
+      if (!skew && p + 4 <= size) {
         *reinterpret_cast<u32*>(out + p) = v;
       } else {
 #pragma unroll
@@ -5107,13 +5102,14 @@ __global__ __launch_bounds__(256) void g_resolve_windows(const State* st, u8* ou
                 kWindowGroups + blockIdx.x % kWindowGroups;
   if (!marks[g]) return;  // uniform; the group lies before the last stripe
   constexpr u32 kPer = (1u << kResolveGroupShift) / 256;
-  const u32 p = u32(g << kResolveGroupShift) + threadIdx.x;
-  u32 r[kPer], mine = 0;
+  const u64 p = (g << kResolveGroupShift) + threadIdx.x;
+  u64 r[kPer];
+  u32 mine = 0;
 #pragma unroll
   for (u32 k = 0; k < kPer; ++k) {
-    const u32 u = p + 256 * k;
+    const u64 u = p + 256 * k;
     const bool unres = (bits[u >> 5] >> (u & 31)) & 1u;
-    r[k] = unres ? roots[u] : 0u;
+    r[k] = unres ? root_position(u, roots[u]) : 0u;
     mine |= u32(unres) << k;
   }
   u32 open = mine;  // chains not at their end
@@ -5130,7 +5126,7 @@ __global__ __launch_bounds__(256) void g_resolve_windows(const State* st, u8* ou
 #pragma unroll
     for (u32 k = 0; k < kPer; ++k) {
       if (!((open >> k) & 1u)) continue;
-      if ((b[k] >> (r[k] & 31)) & 1u) r[k] = n[k];
+      if ((b[k] >> (r[k] & 31)) & 1u) r[k] = root_position(r[k], n[k]);
       else open &= ~(1u << k);
     }
   }
@@ -5138,9 +5134,9 @@ __global__ __launch_bounds__(256) void g_resolve_windows(const State* st, u8* ou
 #pragma unroll
   for (u32 k = 0; k < kPer; ++k) {
     if (!((mine >> k) & 1u)) continue;
-    const u32 u = p + 256 * k;
+    const u64 u = p + 256 * k;
     if (shorten) {
-      __hip_atomic_store(roots + u, r[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      __hip_atomic_store(roots + u, u32(r[k]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     } else {
       const u32 v = out[r[k]];
       out[u] = u8(v);
@@ -5153,12 +5149,12 @@ __global__ __launch_bounds__(256) void g_resolve_windows(const State* st, u8* ou
 
 // The end of a root's chain once the windows are done: a byte of some
 // stripe's window, or one the stripes resolved.
-__device__ __forceinline__ u32 rest_end(const u32* bits, const u32* roots, u32 x, u64 stripe_bytes,
+__device__ __forceinline__ u64 rest_end(const u32* bits, const u32* roots, u64 x, u64 stripe_bytes,
                                         u64 out_end) {
   while ((bits[x >> 5] >> (x & 31)) & 1u) {
     const u64 in = x % stripe_bytes;
     if (in + kStripeWindow >= stripe_bytes && x - in + stripe_bytes < out_end) break;
-    x = roots[x];
+    x = root_position(x, roots[x]);
   }
   return x;
 }
@@ -5214,15 +5210,15 @@ __global__ __launch_bounds__(kRestThreads) void g_resolve_rest(const State* st, 
   const u32 total = listed;
   if (total <= kRestList) {  // uniform
     for (u32 i = t; i < total; i += kRestThreads) {
-      const u32 u = u32(lo) + list[i];
-      const u32 v = out[rest_end(bits, roots, roots[u], stripe_bytes, out_end)];
+      const u64 u = lo + list[i];
+      const u32 v = out[rest_end(bits, roots, root_position(u, roots[u]), stripe_bytes, out_end)];
       out[u] = u8(v);
       as += v;
       aw += (out_end - u) * v;
     }
   } else {
     const bool aligned = (reinterpret_cast<uintptr_t>(out) & 3u) == 0;
-    const u64 w0 = start - kStripeWindow;  // wraps for stripe 0: every root is followed
+    const bool sparse = st->unresolved < out_end / kStripeSparse;  // uniform: roots anywhere
     for (u64 p = lo + 4 * t; p < hi; p += 4 * kRestThreads) {  // a mark group a step
       if (!((marked >> ((p - lo) >> kResolveGroupShift)) & 1u)) continue;
       const u32 nib = (bits[p >> 5] >> (p & 31u)) & 15u;
@@ -5230,16 +5226,18 @@ __global__ __launch_bounds__(kRestThreads) void g_resolve_rest(const State* st, 
       const uint4 rv = *reinterpret_cast<const uint4*>(roots + p);
       const u32 r[4] = {rv.x, rv.y, rv.z, rv.w};
       u32 v = nib == 15u ? 0u : stripe_load4(out, p, out_end, aligned);
-      u32 x[4], b[4], cs = 0, cl = 0;
+      u32 b[4], cs = 0, cl = 0;
+      if (sparse) {
 #pragma unroll
-      for (u32 j = 0; j < 4; ++j) {
-        x[j] = 0;
-        if (!((nib >> j) & 1u)) continue;
-        x[j] = r[j] >= w0 && r[j] < start ? r[j]
-                                          : rest_end(bits, roots, r[j], stripe_bytes, out_end);
+        for (u32 j = 0; j < 4; ++j)
+          if ((nib >> j) & 1u)
+            b[j] = out[rest_end(bits, roots, root_position(p + j, r[j]), stripe_bytes, out_end)];
+      } else {
+        const u8* from = out + start;
+#pragma unroll
+        for (u32 j = 0; j < 4; ++j)
+          b[j] = from[(nib >> j) & 1u ? i32(stripe_offset(start, r[j])) : 0];
       }
-#pragma unroll
-      for (u32 j = 0; j < 4; ++j) b[j] = out[x[j]];
 #pragma unroll
       for (u32 j = 0; j < 4; ++j) {
         if (!((nib >> j) & 1u)) continue;
@@ -5450,9 +5448,9 @@ namespace {
 hipError_t launch_resolve(hipStream_t stream, State* st, u8* out, u32* roots, u32* bits, u8* marks,
                           u64* left, u64 total, u64* parts) {
   if (!total) return hipSuccess;
-  const u64 want = std::min<u64>(kStripes, (total + kStripeMin - 1) / kStripeMin);
-  const u64 stripe = ((total + want - 1) / want + kStripeTile - 1) / kStripeTile * kStripeTile;
-  const u32 stripes = u32((total + stripe - 1) / stripe);
+  const StripeCut cut = cut_stripes(total);
+  const u64 stripe = cut.bytes;
+  const u32 stripes = cut.count;
   HZ_LAUNCH(g_resolve_stripes, dim3(stripes), dim3(kStripeThreads), 0, stream, st, out, roots, bits,
             marks, total, stripe, left, parts);
   HZ_TRY(hipGetLastError());

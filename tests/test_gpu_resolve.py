@@ -99,3 +99,41 @@ def test_resolved_batch(gpu):
     outs = cuda_zlib.decompress_zlib_batch([zlib.compress(r, 9) for r in raws], sizes, gpu)
     for out, raw in zip(outs, raws):
         assert out.cpu().numpy().tobytes() == raw
+
+
+@pytest.mark.parametrize("history", [0, 32768])
+def test_four_gib_output(gpu, history):
+    """The largest output, nearly all of it copied, alone and behind a dictionary
+    (whose window puts its last bytes past 2^32): every byte, and the guard after it."""
+    import ctypes
+    import torch
+    from cuda_zlib import _native
+    total, unit = (1 << 32) - 1, 64 << 20
+    block = np.random.default_rng(9).integers(0, 256, 20011, dtype=np.uint8).tobytes()
+    raw = (block * (unit // len(block) + 1))[:unit]
+    zdict = (block * 2)[-history:] if history else b""
+
+    def piece(data, flush, zdict=b""):
+        c = zlib.compressobj(1, zlib.DEFLATED, -15, 8, 0, *([zdict] if zdict else []))
+        return c.compress(data) + c.flush(flush)
+
+    count = (total + unit - 1) // unit
+    middle = piece(raw, zlib.Z_SYNC_FLUSH)
+    payload = (piece(raw, zlib.Z_SYNC_FLUSH, zdict) + middle * (count - 2) +
+               piece(raw[:total - (count - 1) * unit], zlib.Z_FINISH))
+    lib = _native.load()
+    dev = torch.device("cuda", 0)
+    tensor = lambda b: torch.from_numpy(np.frombuffer(b, np.uint8).copy()).to(dev)
+    src, want, hist = tensor(payload), tensor(raw), tensor(zdict or b"\0")
+    out = torch.full((total + 8,), 0xA5, dtype=torch.uint8, device=dev)
+    meta = torch.zeros(2, dtype=torch.uint32, device=dev)
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    ptr = lambda t: ctypes.c_void_p(t.data_ptr())
+    _native.check(lib, lib.HipZlibDecompressFormat(
+        stream, 1, ptr(hist) if history else None, history, 262144, 262144, ptr(src), len(payload),
+        ptr(out), total, ptr(meta), 2))
+    assert int(meta.cpu().numpy()[0]) == 0
+    for at in range(0, total, unit):
+        n = min(unit, total - at)
+        assert torch.equal(out[at:at + n], want[:n]), at
+    assert (out[total:] == 0xA5).all()

@@ -32,4 +32,12 @@ def test_runs_are_rooted_within_a_back_reference(program):
     root is 1 to 32768 bytes back, and chains have a link per 16 KiB at most."""
     proc = subprocess.run([program, "runs"], capture_output=True, text=True, timeout=600)
     assert proc.returncode == 0, proc.stdout
-    assert "runs checked=75" in proc.stdout
+    assert "runs checked=125" in proc.stdout
+
+
+def test_positions_past_32_bits(program):
+    """Outputs around 2^32 bytes (4 GiB - 1 behind a dictionary's 32 KiB): stripes,
+    roots and the last bytes' stores."""
+    proc = subprocess.run([program, "stripes"], capture_output=True, text=True, timeout=600)
+    assert proc.returncode == 0, proc.stdout
+    assert int(proc.stdout.split("checked=")[1]) > 20000
