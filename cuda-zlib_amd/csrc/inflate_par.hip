@@ -4906,11 +4906,84 @@ struct StripeLoad {
   }
 };
 
-// Below one unresolved byte in this many the stripes are skipped: the chains
-// are few, and following them one by one (g_resolve_windows, g_resolve_rest)
-// costs less than walking the tiles (the 64 MiB strain stream: 57 us
-// against 162).
+// Below one unresolved byte in this many the stripes are skipped: following
+// the chains one by one costs less than walking the tiles (the 64 MiB strain
+// stream: 43 us against 162).
 constexpr u64 kStripeSparse = 64;
+__device__ __forceinline__ bool resolve_sparse(const State* st, u64 out_end) {
+  return st->unresolved < out_end / kStripeSparse;
+}
+
+// With the stripes skipped: one wave follows the chains of mark group g, at most
+// `links` links each, the group's unresolved positions listed in LDS so that
+// every lane has one.  If all end, the group is done; else its bytes stay
+// unresolved, rooted where they got to.  Few unresolved bytes are no short
+// chains: a field that every record copies from the record before has one link
+// a record, 131072 in 64 MiB of 512-byte records.  Passes of kChaseLinks links
+// each leave a chain of n links n / kChaseLinks long or shorter (a root read
+// while it moves is another byte of the same chain), so that the last pass,
+// without limit, has few (16 MiB of such records followed to the end at once:
+// a decode of 5.3 ms, now 3.0).  Returns the bytes left.  Bits never change here,
+// so a
+// chain ends at a byte that emission resolved.
+constexpr u32 kChaseLinks = 64;
+__device__ __forceinline__ u32 chase_group(u8* out, u32* roots, const u32* bits, u64 g, u64 out_end,
+                                           u32 links, u16* list, u64& as, u64& aw) {
+  const u32 lane = lane_id();
+  const u64 base = g << kResolveGroupShift;
+  u32 m = base + 32 * lane < out_end ? bits[(base >> 5) + lane] : 0u;
+  const u32 count = __popc(m), incl = wave_scan_add(count);
+  const u32 total = u32(__builtin_amdgcn_readlane(int(incl), 63));
+  for (u32 at = incl - count; m; m &= m - 1) list[at++] = u16(32 * lane + u32(__builtin_ctz(m)));
+  wave_sync();
+  u64 s = 0, w = 0;
+  bool left = false;
+  for (u32 i = lane; i < total; i += 64) {
+    const u64 u = base + list[i];
+    u64 r = root_position(u, roots[u]);
+    bool ended = false;
+    for (u32 k = 0; k < links && !ended; ++k) {
+      // A link's bit and the root past it load together (of a resolved byte
+      // the root is not used).
+      const u32 b = bits[r >> 5];
+      const u32 n = __hip_atomic_load(roots + r, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      if ((b >> (r & 31)) & 1u) r = root_position(r, n);
+      else ended = true;
+    }
+    if (ended) {
+      const u32 v = out[r];
+      out[u] = u8(v);
+      s += v;
+      w += (out_end - u) * v;
+    } else {
+      __hip_atomic_store(roots + u, u32(r), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      left = true;
+    }
+  }
+  wave_sync();  // the list is rewritten for the next group
+  if (__ballot(left)) return total;
+  as += s;
+  aw += w;
+  if (aw >> 60) aw %= kAdlerMod;
+  return 0;
+}
+
+// chase_group over the marked groups, one per wave, grid-stride; the bytes left
+// are added to *left_count and the marks of finished groups cleared.
+__device__ __forceinline__ void chase_groups(u8* out, u32* roots, const u32* bits, u8* marks,
+                                             u64 out_end, u32 links, u16* list, u64* left_count,
+                                             u64& as, u64& aw) {
+  const u32 waves = blockDim.x / 64, wave = threadIdx.x >> 6;
+  const u64 groups = (out_end + (1u << kResolveGroupShift) - 1) >> kResolveGroupShift;
+  u64 left = 0;
+  for (u64 g = u64(blockIdx.x) * waves + wave; g < groups; g += u64(gridDim.x) * waves) {
+    if (!marks[g]) continue;  // uniform
+    const u32 n = chase_group(out, roots, bits, g, out_end, links, list, as, aw);
+    if (!n && !lane_id()) marks[g] = 0;
+    left += n;
+  }
+  if (left && !lane_id()) atomicAdd(reinterpret_cast<unsigned long long*>(left_count), left);
+}
 
 // Resolves most unresolved bytes: workgroup b walks stripe b of the output in
 // 4 KiB tiles, in order, with the marked tiles of the last 32 KiB of the
@@ -4931,7 +5004,7 @@ g_resolve_stripes(State* st, u8* out, u32* roots, u32* bits, u8* marks, u64 out_
   __shared__ StripeShared sh;
   if (st->status || st->emit_status) return;
   const u32 t = threadIdx.x, lane = lane_id();
-  if (gridDim.x > 1 && st->unresolved < out_end / kStripeSparse) {
+  if (gridDim.x > 1 && resolve_sparse(st, out_end)) {
     if (!blockIdx.x && !t) *left_count = st->unresolved;
     return;
   }
@@ -5096,16 +5169,27 @@ g_resolve_stripes(State* st, u8* out, u32* roots, u32* bits, u8* marks, u64 out_
 // before when most bytes were left (data that repeats itself over many
 // stripes), only the roots move, up to kShortenLinks links along their chains
 // (a root read while it moves is another byte of the same chain).
+// With the stripes skipped, a pass over all bytes (chase_groups): `left` holds
+// the bytes left after the stripes, the first and the second such pass.
 constexpr u32 kShortenLinks = 8;
 constexpr u32 kWindowGroups = kStripeWindow >> kResolveGroupShift;
 __global__ __launch_bounds__(256) void g_resolve_windows(const State* st, u8* out, u32* roots,
-                                                         const u32* bits, const u8* marks,
-                                                         u64 out_end, u64 stripe_bytes,
-                                                         const u64* left_count, u32 shorten,
+                                                         const u32* bits, u8* marks, u64 out_end,
+                                                         u64 stripe_bytes, u64* left,
+                                                         u32 chase_from, u32 chase_to, u32 shorten,
                                                          u64* parts) {
   __shared__ u64 red[2][16];
-  if (st->status || st->emit_status || !*left_count) return;
-  if (shorten && *left_count < out_end / 2) return;
+  __shared__ u16 list[256 / 64][1 << kResolveGroupShift];
+  if (st->status || st->emit_status) return;
+  if (resolve_sparse(st, out_end)) {  // uniform
+    if (!left[chase_from]) return;
+    u64 as = 0, aw = 0;
+    chase_groups(out, roots, bits, marks, out_end, kChaseLinks, list[threadIdx.x >> 6],
+                 &left[chase_to], as, aw);
+    if (parts) resolve_add_parts(parts, as, aw, red);
+    return;
+  }
+  if (!*left || (shorten && *left < out_end / 2)) return;
   const u64 g = ((blockIdx.x / kWindowGroups + 1) * stripe_bytes >> kResolveGroupShift) -
                 kWindowGroups + blockIdx.x % kWindowGroups;
   if (!marks[g]) return;  // uniform; the group lies before the last stripe
@@ -5155,38 +5239,38 @@ __global__ __launch_bounds__(256) void g_resolve_windows(const State* st, u8* ou
   if (parts && !shorten) resolve_add_parts(parts, as, aw, red);
 }
 
-// The end of a root's chain once the windows are done: a byte of some
-// stripe's window, or one the stripes resolved.
-__device__ __forceinline__ u64 rest_end(const u32* bits, const u32* roots, u64 x, u64 stripe_bytes,
-                                        u64 out_end) {
-  while ((bits[x >> 5] >> (x & 31)) & 1u) {
-    const u64 in = x % stripe_bytes;
-    if (in + kStripeWindow >= stripe_bytes && x - in + stripe_bytes < out_end) break;
-    x = root_position(x, roots[x]);
-  }
-  return x;
-}
-
 // The other bytes g_resolve_stripes left: their roots lie in the 32 KiB before
-// their stripe (final by now), or elsewhere (with the stripes skipped) and are
-// followed.  A workgroup sweeps kRestBytes of a stripe: with
+// their stripe, final by now.  A workgroup sweeps kRestBytes of a stripe: with
 // few bytes left there it lists them and takes one a thread, else four
-// consecutive positions a thread.
+// consecutive positions a thread.  With the stripes skipped, the chains that the
+// passes before left, to their ends.
 constexpr u32 kXcds = 8;  // MI355X: 8 accelerator complex dies of 32 CUs
 constexpr u32 kRestThreads = 512;
 constexpr u32 kRestBytes = 16384;
 constexpr u32 kRestList = 4 * kRestThreads;
 static_assert(4 * kRestThreads == 1u << kResolveGroupShift, "a step is a mark group");
-__global__ __launch_bounds__(kRestThreads) void g_resolve_rest(const State* st, u8* out,
-                                                               const u32* roots, const u32* bits,
-                                                               const u8* marks, u64 out_end,
-                                                               u64 stripe_bytes, u32 parts_per,
-                                                               const u64* left_count, u64* parts) {
+__global__ __launch_bounds__(kRestThreads) void g_resolve_rest(const State* st, u8* out, u32* roots,
+                                                               const u32* bits, u8* marks,
+                                                               u64 out_end, u64 stripe_bytes,
+                                                               u32 parts_per, u64* left, u64* parts) {
   __shared__ u64 red[2][16];
-  __shared__ u16 list[kRestList];
+  union Lists {
+    u16 stripe[kRestList];
+    u16 wave[kRestThreads / 64][1 << kResolveGroupShift];
+  };
+  __shared__ Lists lists;
   __shared__ u32 listed;
-  if (st->status || st->emit_status || !*left_count) return;
+  if (st->status || st->emit_status) return;
   const u32 t = threadIdx.x, lane = lane_id();
+  u64 as = 0, aw = 0;
+  if (resolve_sparse(st, out_end)) {  // uniform
+    if (!left[2]) return;
+    chase_groups(out, roots, bits, marks, out_end, ~0u, lists.wave[t >> 6], &left[3], as, aw);
+    if (parts) resolve_add_parts(parts, as, aw, red);
+    return;
+  }
+  if (!*left) return;
+  u16* list = lists.stripe;
   // Workgroups go to the 8 XCDs in turn: a stripe's stay on one, whose L2
   // then holds the window they read.
   const u32 slot = blockIdx.x / kXcds;
@@ -5204,7 +5288,7 @@ __global__ __launch_bounds__(kRestThreads) void g_resolve_rest(const State* st, 
   if (!marked) return;  // uniform
   if (!t) listed = 0;
   __syncthreads();
-  u64 as = 0, aw = 0;
+  const u8* from = out + start;
   // Two bitmap words a thread (hi is a multiple of 4096 or the output's end,
   // whose bitmap has a word more).
   const u32 w = 2 * t;
@@ -5219,14 +5303,13 @@ __global__ __launch_bounds__(kRestThreads) void g_resolve_rest(const State* st, 
   if (total <= kRestList) {  // uniform
     for (u32 i = t; i < total; i += kRestThreads) {
       const u64 u = lo + list[i];
-      const u32 v = out[rest_end(bits, roots, root_position(u, roots[u]), stripe_bytes, out_end)];
+      const u32 v = from[i32(stripe_offset(start, roots[u]))];
       out[u] = u8(v);
       as += v;
       aw += (out_end - u) * v;
     }
   } else {
     const bool aligned = (reinterpret_cast<uintptr_t>(out) & 3u) == 0;
-    const bool sparse = st->unresolved < out_end / kStripeSparse;  // uniform: roots anywhere
     for (u64 p = lo + 4 * t; p < hi; p += 4 * kRestThreads) {  // a mark group a step
       if (!((marked >> ((p - lo) >> kResolveGroupShift)) & 1u)) continue;
       const u32 nib = (bits[p >> 5] >> (p & 31u)) & 15u;
@@ -5235,17 +5318,8 @@ __global__ __launch_bounds__(kRestThreads) void g_resolve_rest(const State* st, 
       const u32 r[4] = {rv.x, rv.y, rv.z, rv.w};
       u32 v = nib == 15u ? 0u : stripe_load4(out, p, out_end, aligned);
       u32 b[4], cs = 0, cl = 0;
-      if (sparse) {
 #pragma unroll
-        for (u32 j = 0; j < 4; ++j)
-          if ((nib >> j) & 1u)
-            b[j] = out[rest_end(bits, roots, root_position(p + j, r[j]), stripe_bytes, out_end)];
-      } else {
-        const u8* from = out + start;
-#pragma unroll
-        for (u32 j = 0; j < 4; ++j)
-          b[j] = from[(nib >> j) & 1u ? i32(stripe_offset(start, r[j])) : 0];
-      }
+      for (u32 j = 0; j < 4; ++j) b[j] = from[(nib >> j) & 1u ? i32(stripe_offset(start, r[j])) : 0];
 #pragma unroll
       for (u32 j = 0; j < 4; ++j) {
         if (!((nib >> j) & 1u)) continue;
@@ -5452,7 +5526,8 @@ u32 clamp_grid(u64 want, u32 cap) { return u32(want < 1 ? 1 : (want > cap ? cap 
 namespace {
 // Resolution of the unresolved bytes of out[0, total): the stripes, then the
 // bytes they leave, first those in the stripes' windows.  With one stripe
-// nothing is left.  left: a zeroed counter.
+// nothing is left.  left: kResolveCounts zeroed counters.
+constexpr u32 kResolveCounts = 4;
 hipError_t launch_resolve(hipStream_t stream, State* st, u8* out, u32* roots, u32* bits, u8* marks,
                           u64* left, u64 total, u64* parts) {
   if (!total) return hipSuccess;
@@ -5463,11 +5538,13 @@ hipError_t launch_resolve(hipStream_t stream, State* st, u8* out, u32* roots, u3
             marks, total, stripe, left, parts);
   HZ_TRY(hipGetLastError());
   if (stripes == 1) return hipSuccess;
+  u32 chased = 0;  // the counter of the pass before
   for (u32 shorten = stripes > kShortenLinks ? 1 : 0;; shorten = 0) {
     HZ_LAUNCH(g_resolve_windows, dim3((stripes - 1) * kWindowGroups), dim3(256), 0, stream, st, out,
-              roots, bits, marks, total, stripe, left, shorten, parts);
+              roots, bits, marks, total, stripe, left, chased, shorten ? 1u : 2u, shorten, parts);
     HZ_TRY(hipGetLastError());
     if (!shorten) break;
+    chased = 1;
   }
   const u32 per = u32((stripe + kRestBytes - 1) / kRestBytes);
   HZ_LAUNCH(g_resolve_rest, dim3((stripes + kXcds - 1) / kXcds * kXcds * per), dim3(kRestThreads),
@@ -5503,10 +5580,10 @@ hipError_t run_inflate_general(hipStream_t stream, Scratch& scratch, const u8* i
   const u64 need_words = tiles / 32 + 1;
   // Adler-32 partial pairs: kAdlerSlots each for the lane emitter, the
   // serial emitter and the resolve kernels (workgroups add theirs, so they
-  // start at zero), summed by g_finish.  The pairs, the count of bytes left and the
+  // start at zero), summed by g_finish.  The pairs, the counts of bytes left and the
   // unresolved bitmap are zeroed by g_frame.
   u8* zeroed = nullptr;
-  const u64 zero_u64 = 2 * u64(3 * kAdlerSlots) + 1;
+  const u64 zero_u64 = 2 * u64(3 * kAdlerSlots) + kResolveCounts;
   // Resolve group marks (emission marks groups in marks0).
   const u64 mark_groups_n = (words + 63) / 64;
   const u64 zero_bytes = 8 * zero_u64 + 4 * words + 4 * need_words + (mark_groups_n + 3) / 4 * 4;
@@ -5663,7 +5740,7 @@ hipError_t run_inflate_general(hipStream_t stream, Scratch& scratch, const u8* i
   const u32 emit_grid = clamp_grid(std::min<u64>(max_blocks, items_cap), 4096);
   u64* adler_parts = reinterpret_cast<u64*>(zeroed);
   u64* left = adler_parts + 2 * u64(3 * kAdlerSlots);
-  u32* bits0 = reinterpret_cast<u32*>(left + 1);
+  u32* bits0 = reinterpret_cast<u32*>(left + kResolveCounts);
   u8* marks0 = zeroed + 8 * zero_u64 + 4 * words + 4 * need_words;
   const u64 out_end = out_total;  // a byte at position p is stream byte n - (out_end - p)
   // Emission by segments, then the queued units of long fixed runs.
@@ -5716,10 +5793,10 @@ hipError_t run_inflate_batch_wide(hipStream_t stream, Scratch& scratch, const u8
                              in_bits / (u64(kDescThreads) * kDescMinSlice) + 8 * u64(n) + 64;
   const u64 words = (out_total + 31) / 32 + 1;
   const u64 mark_groups_n = (words + 63) / 64;
-  // The state, the count of bytes the stripes leave, the bitmap and its group marks start
+  // The state, the counts of bytes left, the bitmap and its group marks start
   // zeroed: one allocation, cleared by one fill.
   const u64 st_bytes = scratch_round(sizeof(State));
-  const u64 left_bytes = scratch_round(sizeof(u64));
+  const u64 left_bytes = scratch_round(kResolveCounts * sizeof(u64));
   const u64 zero_bytes = st_bytes + left_bytes + words * 4 + mark_groups_n;
   u8* zeroed = nullptr;
   HZ_TRY(scratch.alloc(&zeroed, zero_bytes));

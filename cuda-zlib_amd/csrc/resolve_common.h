@@ -14,7 +14,8 @@ constexpr u32 kNoRoot = 0xffffffffu;  // handed down by emission: a resolved byt
 
 // Positions take more than 32 bits (an output of up to 2^32 - 1 bytes behind a
 // dictionary's window), roots are kept in 32: the low bits of a position less
-// than 2^32 bytes before the byte at p.
+// than 2^32 bytes before the byte at p.  (Roots moved along their chains are of
+// unresolved bytes, which lie in the output, not in the window before it.)
 __host__ __device__ __forceinline__ u64 root_position(u64 p, u32 root) {
   return p - u32(u32(p) - root);
 }
