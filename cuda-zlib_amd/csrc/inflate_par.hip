@@ -427,7 +427,8 @@ constexpr u32 kSurvivorCap = 1024;  // prefilter survivors a wave checks per pas
 using PreStage = StageT<kPreStageWords>;
 // Pre-candidate entries: bit offset, plus this flag once the header is known valid.
 constexpr u64 kValidBit = 1ull << 62;
-constexpr u64 kPosMask = kValidBit - 1;
+constexpr u64 kStoredBit = 1ull << 61;  // a stored block's header
+constexpr u64 kPosMask = kStoredBit - 1;
 constexpr u32 kKindShift = 30;  // wg_count: count | kind << 30
 constexpr u32 kCountMask = (1u << kKindShift) - 1;
 
@@ -885,7 +886,8 @@ __global__ __launch_bounds__(256) void g_discover(const u8* body, u64 len, State
       while (mask) {
         const u32 k = __builtin_ctzll(mask);
         mask &= mask - 1;
-        wg_list[wg * kDiscCap + base++] = (b0 * 8 + k) | ((valid_flag >> k) & 1 ? kValidBit : 0);
+        wg_list[wg * kDiscCap + base++] = (b0 * 8 + k) | ((valid_flag >> k) & 1 ? kValidBit : 0) |
+                                          ((stored_flag >> k) & 1 ? kStoredBit : 0);
       }
     }
     __syncthreads();  // the next range reuses the stage and the lists
@@ -1364,13 +1366,22 @@ __global__ __launch_bounds__(64) void g_validate(const u8* body, u64 len, State*
 // the workgroup holding the last entry sets the candidate count and checks
 // the candidate limit (valid headers + bit 0 + stored seeds, as the
 // reference counts them).
+// Candidates have the decode-table slot of their index.  Where stored blocks
+// are among them (which need none, and could use all slots up: 16 MiB of 2 KB
+// stored blocks before 32 MiB of text), the others take slots in any order:
+// slots maps candidates to them, slot_pos slots to header bits.
 __global__ __launch_bounds__(256) void g_valid_scatter(State* st, const u64* pre,
                                                        const u32* wave_valid, u64* cand,
-                                                       u64 cand_capacity, u64 max_candidates) {
+                                                       u64 cand_capacity, u64 max_candidates,
+                                                       u32* slots, u64* slot_pos,
+                                                       u64 table_capacity) {
   static_assert(kDiscThreads % kValPerWave == 0, "a block covers whole validation waves");
   __shared__ u32 wave_count[kDiscThreads / 64];
+  __shared__ u32 wave_coded[kDiscThreads / 64];
   __shared__ u64 red[kDiscThreads / 64];
+  __shared__ u64 first_slot;
   if (st->status) return;
+  const bool mapped = st->stored != 0;
   const u64 n = st->precount;
   if (u64(blockIdx.x) * kDiscThreads >= n) return;
   const u32 t = threadIdx.x, wave = t >> 6, lane = lane_id();
@@ -1389,23 +1400,44 @@ __global__ __launch_bounds__(256) void g_valid_scatter(State* st, const u64* pre
   const u64 i = u64(blockIdx.x) * kDiscThreads + t;
   const u64 e = i < n ? pre[i] : 0;
   const bool valid = i < n && (e & kValidBit);
-  const u64 bal = __ballot(valid);
+  const u64 bal = __ballot(valid), coded = __ballot(valid && !(e & kStoredBit));
   if (!lane) {
     wave_count[wave] = __popcll(bal);
+    wave_coded[wave] = __popcll(coded);
     red[wave] = part;
   }
   __syncthreads();
+  if (mapped) {  // uniform
+    if (!t) {
+      u32 n_coded = 0;
+      for (u32 w = 0; w < kDiscThreads / 64; ++w) n_coded += wave_coded[w];
+      if (n_coded)
+        first_slot = atomicAdd(reinterpret_cast<unsigned long long*>(&st->tables_used), u64(n_coded));
+    }
+    __syncthreads();
+  }
   u64 at = 0;
   for (u32 w = 0; w < kDiscThreads / 64; ++w) at += red[w];
   const u64 block_base = at;
   for (u32 w = 0; w < wave; ++w) at += wave_count[w];
   at += __popcll(bal & lanemask_lt());
-  if (valid && at < cand_capacity) cand[at] = e & kPosMask;
+  if (valid && at < cand_capacity) {
+    cand[at] = e & kPosMask;
+    if (mapped) {
+      u64 slot = kNone;
+      if (!(e & kStoredBit)) {
+        slot = first_slot + __popcll(coded & lanemask_lt());
+        for (u32 w = 0; w < wave; ++w) slot += wave_coded[w];
+        if (slot < table_capacity) slot_pos[slot] = e & kPosMask;
+      }
+      slots[at] = u32(slot);
+    }
+  }
   if (!t && (u64(blockIdx.x) + 1) * kDiscThreads >= n) {
     u64 total = block_base;
     for (u32 w = 0; w < kDiscThreads / 64; ++w) total += wave_count[w];
     st->candidates = total;
-    st->tables_used = total;  // table slots 0 .. total-1 belong to the candidates
+    if (!mapped) st->tables_used = total;  // table slots 0 .. total-1 belong to the candidates
     if (total - st->stored + st->seeds > max_candidates) st->status = kCandidateOverflow;
   }
 }
@@ -2359,21 +2391,23 @@ struct HeaderShared {
 
 }  // namespace
 
-// One wave per candidate (below the table capacity): parse its dynamic
+// One wave per candidate with a table slot: parse its dynamic
 // header, build the literal/length and distance tables in the fast format
-// into the candidate's table slot, and record the first token bit and flags
+// into the slot, and record the first token bit and flags
 // (hdr_info: status | BFINAL << 8 | BTYPE << 9).  Bit 0 is a candidate
 // whatever its block type: a stored or fixed block there is only recorded
 // (BTYPE != 2, no tables) and g_describe parses it itself.
 __global__ __launch_bounds__(64) void g_headers(const u8* body, u64 len, const State* st,
-                                                const u64* cand, BlockTables* tables,
-                                                u64 table_capacity, u64* hdr_d0, u32* hdr_info) {
+                                                const u64* cand, const u64* slot_pos,
+                                                BlockTables* tables, u64 table_capacity,
+                                                u64* hdr_d0, u32* hdr_info) {
   __shared__ HeaderShared sh;
   if (st->status) return;
   const u32 lane = threadIdx.x;
-  const u64 n = min<u64>(st->candidates, table_capacity);
+  const u64 n = min<u64>(st->tables_used, table_capacity);
+  const u64* headers = st->stored ? slot_pos : cand;  // by slot
   for (u64 c = blockIdx.x; c < n; c += gridDim.x) {
-    const u64 pos = cand[c];
+    const u64 pos = headers[c];
     stage_range(body, len, pos, pos + 8, sh.stage, kHeaderBytes);
     __syncthreads();
     // Lane 0 reads BFINAL and BTYPE; the wave reads the fields and the
@@ -2482,12 +2516,13 @@ __global__ __launch_bounds__(kDescThreads) void g_describe(
     const u8* body, u64 len, const u64* cand, State* st, u64 out_size, u64* seg_end,
     u64* seg_size, u32* seg_blocks, u32* seg_next, u32* seg_flags, u32* seg_rec, BlockRec* recs,
     u64 rec_capacity, u64* slice_entry, u32* slice_off, u32* group_link, u64 group_capacity,
-    BlockTables* tables, u64 table_capacity, const u64* hdr_d0, const u32* hdr_info,
-    u32* seg_last, u32* region_cand) {
+    BlockTables* tables, u64 table_capacity, const u32* slots, const u64* hdr_d0,
+    const u32* hdr_info, u32* seg_last, u32* region_cand) {
   __shared__ DescShared sh;
   if (st->status) return;
   const u32 t = threadIdx.x;
   const u64 n = st->candidates;
+  const bool mapped = st->stored != 0;
   for (u64 c = blockIdx.x; c < n; c += gridDim.x) {
     u64 produced = 0;
     u32 blocks = 0, status = 0, final_block = 0, next = kNone, first_rec = kNone, last_rec = kNone;
@@ -2497,10 +2532,11 @@ __global__ __launch_bounds__(kDescThreads) void g_describe(
     u64 search_from = c + 1;
     bool recs_ok = true;
     // The candidate's own dynamic header was parsed by g_headers (tables in
-    // slot c); any other block type at bit 0 is parsed below.  Its position,
+    // its slot); a stored block, or any type at bit 0, is parsed below.  Its position,
     // header results and tables load at once (one memory latency).
-    const u32 info0 = c < table_capacity ? hdr_info[c] : 0u;
-    const bool pre0 = c < table_capacity && ((info0 >> 9) & 3u) == 2;
+    const u64 slot = mapped ? u64(slots[c]) : c;
+    const u32 info0 = slot < table_capacity ? hdr_info[slot] : 0u;
+    const bool pre0 = slot < table_capacity && ((info0 >> 9) & 3u) == 2;
     if (!t) {
       sh.pos = cand[c];
       sh.stage.count = 0;
@@ -2509,12 +2545,12 @@ __global__ __launch_bounds__(kDescThreads) void g_describe(
         sh.status = info0 & 0xffu;
         sh.final_block = (info0 >> 8) & 1u;
         sh.type = (info0 >> 9) & 3u;
-        sh.d0 = hdr_d0[c];
+        sh.d0 = hdr_d0[slot];
       }
     }
     if (pre0) {
-      const u32* src_ll = reinterpret_cast<const u32*>(&tables[c].ll);
-      const u32* src_dd = reinterpret_cast<const u32*>(&tables[c].dd);
+      const u32* src_ll = reinterpret_cast<const u32*>(&tables[slot].ll);
+      const u32* src_dd = reinterpret_cast<const u32*>(&tables[slot].dd);
       u32* dst_ll = reinterpret_cast<u32*>(&sh.tables.ll);
       u32* dst_dd = reinterpret_cast<u32*>(&sh.tables.dd);
       copy_tables<kDescThreads>(dst_ll, dst_dd, src_ll, src_dd, t);
@@ -2558,7 +2594,7 @@ __global__ __launch_bounds__(kDescThreads) void g_describe(
         sh.hint = idx < n ? cand[idx] : len * 8;
         sh.group = kNone;
         sh.lanes = 0;
-        if (pre) sh.table = u32(c);
+        if (pre) sh.table = u32(slot);
         else {
           const u64 ti = atomicAdd(reinterpret_cast<unsigned long long*>(&st->tables_used), 1ull);
           sh.table = ti < table_capacity ? u32(ti) : kNone;
@@ -5617,6 +5653,8 @@ hipError_t run_inflate_general(hipStream_t stream, Scratch& scratch, const u8* i
   u64 *seg_end = nullptr, *seg_size = nullptr, *hdr_d0 = nullptr;
   u32 *seg_blocks = nullptr, *seg_next = nullptr, *seg_flags = nullptr, *exit_node = nullptr;
   u32 *seg_rec = nullptr, *seg_last = nullptr, *region_cand = nullptr, *hdr_info = nullptr;
+  u32* slots = nullptr;
+  u64* slot_pos = nullptr;
   FixSummary* fix_sum = nullptr;
   uint2* fix_entries = nullptr;
   FixRun* fix_runs = nullptr;
@@ -5642,6 +5680,8 @@ hipError_t run_inflate_general(hipStream_t stream, Scratch& scratch, const u8* i
     HZ_TRY(s.alloc(&region_cand, cand_capacity));
     HZ_TRY(s.alloc(&hdr_d0, table_capacity));
     HZ_TRY(s.alloc(&hdr_info, table_capacity));
+    HZ_TRY(s.alloc(&slots, cand_capacity));
+    HZ_TRY(s.alloc(&slot_pos, table_capacity));
     HZ_TRY(s.alloc(&fix_sum, tiles * kFixEntries));
     HZ_TRY(s.alloc(&fix_entries, tiles));
     HZ_TRY(s.alloc(&fix_runs, run_capacity));
@@ -5672,7 +5712,7 @@ hipError_t run_inflate_general(hipStream_t stream, Scratch& scratch, const u8* i
             wave_valid);
   HZ_TRY(hipGetLastError());
   HZ_LAUNCH(g_valid_scatter, dim3(u32(pre_blocks)), dim3(kDiscThreads), 0, stream, st, pre,
-            wave_valid, cand, cand_capacity, u64(max_candidates));
+            wave_valid, cand, cand_capacity, u64(max_candidates), slots, slot_pos, table_capacity);
   HZ_TRY(hipGetLastError());
 
   // Describe every candidate's segment.
@@ -5689,7 +5729,7 @@ hipError_t run_inflate_general(hipStream_t stream, Scratch& scratch, const u8* i
   // them, and idle workgroups of a 4096-wide launch cost their dispatch.
   const u64 items_cap = std::max<u64>(256, len / 64);
   HZ_LAUNCH(g_headers, dim3(clamp_grid(std::min(table_capacity, 2 * items_cap), 8192)), dim3(kWave), 0, stream, body, len, st,
-            cand, tables, table_capacity, hdr_d0, hdr_info);
+            cand, slot_pos, tables, table_capacity, hdr_d0, hdr_info);
   HZ_TRY(hipGetLastError());
   HZ_TRY(scratch.alloc(&slice_entry, group_capacity * 64));
   HZ_TRY(scratch.alloc(&slice_off, group_capacity * 64));
@@ -5698,7 +5738,7 @@ hipError_t run_inflate_general(hipStream_t stream, Scratch& scratch, const u8* i
   HZ_LAUNCH(g_describe, dim3(clamp_grid(std::min(cand_capacity, items_cap), 4096)), dim3(kDescThreads), 0, stream, body, len,
             cand, st, out_size, seg_end, seg_size, seg_blocks, seg_next, seg_flags, seg_rec, recs,
             rec_capacity, slice_entry, slice_off, group_link, group_capacity, tables,
-            table_capacity, hdr_d0, hdr_info, seg_last, region_cand);
+            table_capacity, slots, hdr_d0, hdr_info, seg_last, region_cand);
   HZ_TRY(hipGetLastError());
   HZ_LAUNCH(g_fix_mark, dim3(1), dim3(256), 0, stream, st, cand, len, seg_end, seg_flags,
             region_cand, fix_need, tiles);

@@ -68,6 +68,31 @@ def test_broken_chain(gpu, cut):
         assert (status, got) == (want_status, want)
 
 
+@pytest.mark.parametrize("block", [1500, 2043, 4000])
+@pytest.mark.parametrize("order", ["stored first", "stored last", "mixed"])
+def test_more_stored_candidates_than_table_slots(gpu, block, order):
+    """Thousands of short stored blocks and hundreds of dynamic ones (memLevel 1), whose
+    decode tables have a slot per 8 KiB of the stream and 1024 more."""
+    noise = _random(7 << 20, block)
+    stored = [(_stored(noise[i:i + block]), noise[i:i + block]) for i in range(0, len(noise), block)]
+    texts = []
+    for i in range(8):
+        text = workloads.text_like(256 * KIB, np.random.default_rng(i))
+        c = zlib.compressobj(6, zlib.DEFLATED, -15, 1)
+        texts.append((c.compress(text) + c.flush(zlib.Z_FULL_FLUSH), text))
+    if order == "mixed":
+        step = len(stored) // len(texts) + 1
+        parts = [p for i, t in enumerate(texts) for p in stored[i * step:(i + 1) * step] + [t]]
+    else:
+        parts = stored + texts if order == "stored first" else texts + stored
+    data = b"".join(raw for _, raw in parts)
+    stream = _wrap(b"".join(coded for coded, _ in parts) + _stored(b"end", True), data + b"end")
+    assert zlib.decompress(stream) == data + b"end"
+    got, status, _ = capi_decompress(stream, len(data) + 3)
+    assert status == 0
+    assert got == data + b"end"
+
+
 @pytest.mark.parametrize("tail", [120, 300, 520, 640, 700, 1000])
 @pytest.mark.parametrize("size", [30 * KIB, 900 * KIB])
 def test_last_header_near_the_end(gpu, size, tail):
