@@ -2707,10 +2707,17 @@ __global__ __launch_bounds__(256) void g_fix_mark(const State* st, const u64* ca
         break;
       }
     }
-    // To the end of its group, so that the walk takes the run's end in one step.
-    const u64 last = (h / kFixTileBits) | (kFixGroupTiles - 1);
-    if (tiles) fix_mark_tiles(fix_need, x / kFixTileBits / kFixGroupTiles * kFixGroupTiles,
-                              min<u64>(last, tiles - 1));
+    // A region of a group's tiles or more takes whole groups, so that the walk
+    // starts and ends in group steps (at most twice the tiles marked); a shorter
+    // one is walked tile by tile.  (With groups for every region, a fixed block
+    // of 200 bytes per 128 KiB of text had half the body summarised: 16 MiB
+    // 1347 us, now 1162.)
+    u64 k0 = x / kFixTileBits, k1 = h / kFixTileBits;
+    if (k1 - k0 >= kFixGroupTiles) {
+      k0 = k0 / kFixGroupTiles * kFixGroupTiles;
+      k1 |= kFixGroupTiles - 1;
+    }
+    if (tiles) fix_mark_tiles(fix_need, k0, min<u64>(k1, tiles - 1));
   }
 }
 

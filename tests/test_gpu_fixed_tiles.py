@@ -137,3 +137,27 @@ def test_second_walk_over_a_run(gpu, no_cpu_codec, seed):
         out, meta = cuda_zlib.decompress_zlib_checked(stream, len(data), 0)
     assert int(meta.cpu().numpy()[0]) == 0
     assert out.cpu().numpy().tobytes() == data
+
+
+@pytest.mark.parametrize("length", [100, 200, 600, 5000, 60000, 66000, 200003])
+@pytest.mark.parametrize("gap", [3000, 70000, 131072])
+def test_fixed_blocks_between_dynamic_ones(gpu, length, gap):
+    """Fixed blocks of literals shorter and longer than a group of tiles, each between
+    dynamic blocks and one at the end of the body."""
+    rng = np.random.default_rng(length + gap)
+
+    def piece(data, strategy, flush=zlib.Z_FULL_FLUSH):
+        c = zlib.compressobj(6, zlib.DEFLATED, -15, 8, strategy)
+        return c.compress(data) + c.flush(flush)
+
+    body = raw = b""
+    for i in range(6):
+        text = workloads.text_like(gap, rng)
+        literals = rng.integers(48, 91, length, dtype=np.uint8).tobytes()
+        fixed = piece(literals, zlib.Z_FIXED, zlib.Z_FINISH if i == 5 else zlib.Z_FULL_FLUSH)
+        assert (fixed[0] >> 1) & 3 == 1
+        body += piece(text, zlib.Z_DEFAULT_STRATEGY) + fixed
+        raw += text + literals
+    stream = b"\x78\x9c" + body + zlib.adler32(raw).to_bytes(4, "big")
+    assert zlib.decompress(stream) == raw
+    _check(gpu, stream, raw, length % 4)
