@@ -2711,7 +2711,7 @@ __global__ __launch_bounds__(256) void g_fix_mark(const State* st, const u64* ca
     // starts and ends in group steps (at most twice the tiles marked); a shorter
     // one is walked tile by tile.  (With groups for every region, a fixed block
     // of 200 bytes per 128 KiB of text had half the body summarised: 16 MiB
-    // 1347 us, now 1162.)
+    // 1347 us against 1162.)
     u64 k0 = x / kFixTileBits, k1 = h / kFixTileBits;
     if (k1 - k0 >= kFixGroupTiles) {
       k0 = k0 / kFixGroupTiles * kFixGroupTiles;
@@ -2997,6 +2997,30 @@ __global__ __launch_bounds__(256) void g_fix_groups(const State* st, const u32* 
   }
 }
 
+namespace {
+
+// f(i) for this workgroup's slots of more than one tile (slot i is workgroup
+// i mod gridDim.x's), looked for by all threads at once: a walk takes slots 64
+// at a time, and with many short runs nearly all are unused (one load after
+// the other, 128 runs took g_fix_slices 182 us, now 91, g_fix_expand 19, now 5).
+template <class F>
+__device__ __forceinline__ void for_group_slots(const FixTile* rt, u64 used, const F& f) {
+  __shared__ u32 list[kFixThreads];
+  __shared__ u32 listed;
+  for (u64 i0 = blockIdx.x; i0 < used; i0 += u64(kFixThreads) * gridDim.x) {
+    if (!threadIdx.x) listed = 0;
+    __syncthreads();
+    const u64 i = i0 + u64(threadIdx.x) * gridDim.x;
+    if (i < used && rt[i].run != kNone && rt[i].tiles > 1) list[atomicAdd(&listed, 1u)] = u32(i);
+    __syncthreads();
+    const u32 n = listed;
+    for (u32 q = 0; q < n; ++q) f(u64(list[q]));
+    __syncthreads();  // the list is refilled next
+  }
+}
+
+}  // namespace
+
 // The true entries of the tiles a walk stepped over in groups: per slot of
 // more than one tile, the entry bit (low 5 bits of x), the slot (the rest) and
 // the run's output bytes before (y) of every tile after the first, at the
@@ -3010,9 +3034,8 @@ __global__ __launch_bounds__(256) void g_fix_expand(const State* st, const FixTi
   __shared__ FixSummary all[kFixGroupTiles][kFixEntries];
   if (st->status || !st->fix_regions) return;
   const u64 used = min<u64>(st->fix_rt, rt_capacity);
-  for (u64 i = blockIdx.x; i < used; i += gridDim.x) {
+  for_group_slots(rt, used, [&](u64 i) {
     const FixTile ft = rt[i];
-    if (ft.run == kNone || ft.tiles < 2) continue;  // uniform
     const uint4* src = reinterpret_cast<const uint4*>(sum + u64(ft.k) * kFixEntries);
     for (u32 q = threadIdx.x; q < ft.tiles * kFixEntries; q += 256)
       reinterpret_cast<uint4*>(&all[0][0])[q] = src[q];
@@ -3029,7 +3052,7 @@ __global__ __launch_bounds__(256) void g_fix_expand(const State* st, const FixTi
       if (threadIdx.x && threadIdx.x < ft.tiles) entries[u64(ft.k) + threadIdx.x] = mine;
     }
     __syncthreads();
-  }
+  });
 }
 
 namespace {
@@ -3426,10 +3449,10 @@ __global__ __launch_bounds__(kFixThreads) void g_fix_slices(const u8* body, u64 
   };
   // Tile blockIdx.y of the slots of many tiles, then the slots of one tile
   // dealt over the whole grid.
-  for (u64 i = blockIdx.x; i < used; i += gridDim.x) {
+  for_group_slots(rt, used, [&](u64 i) {
     const FixTile ft = rt[i];
-    if (ft.run < nruns && ft.tiles > 1 && blockIdx.y < ft.tiles) tile(ft, i, blockIdx.y);  // uniform
-  }
+    if (ft.run < nruns && blockIdx.y < ft.tiles) tile(ft, i, blockIdx.y);  // uniform
+  });
   for (u64 i = blockIdx.x + u64(gridDim.x) * blockIdx.y; i < used;
        i += u64(gridDim.x) * gridDim.y) {
     const FixTile ft = rt[i];
