@@ -1092,6 +1092,61 @@ __host__ __device__ __forceinline__ u32 fixed_token(u64 b, u32& nbits, u32& leng
   return kKindLen;
 }
 
+// The token of a fixed-Huffman block at the low bits of `b` as a 16-bit step,
+// without branches, from an entry of fixed_step_entry for its first 9 bits:
+// twice the bits taken | the output bytes << 6 for a token; no bits for a
+// special, whose value is kStepEob | the next header's three bits (| 8 if they
+// are cut off) or an error's status.
+constexpr u32 kStepEob = 16;
+// x's `width` bits from bit `offset` on (the low five bits of each).
+__host__ __device__ __forceinline__ u32 bit_field(u32 x, u32 offset, u32 width) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __builtin_amdgcn_ubfe(x, offset, width);
+#else
+  return (x >> (offset & 31u)) & ((1u << (width & 31u)) - 1u);
+#endif
+}
+// Of the next 9 bits: where the length's extra bits start (bits 0-4), their
+// number (5-9), the bits before a distance (10-14), the length's base
+// (15-23), a distance follows (31).  An EOB takes the header's bits for extra
+// ones.
+__host__ __device__ __forceinline__ u32 fixed_step_entry(u32 i) {
+  const u32 r9 = __builtin_bitreverse32(i) >> 23;
+  u32 sym, l;
+  if ((r9 >> 2) < 24) {
+    sym = 256 + (r9 >> 2);
+    l = 7;
+  } else if ((r9 >> 1) < 0xC8) {
+    sym = (r9 >> 1) < 0xC0 ? (r9 >> 1) - 0x30 : (r9 >> 1) + 88;  // 0xC0 -> 280
+    l = 8;
+  } else {
+    sym = r9 - 256;
+    l = 9;
+  }
+  if (sym < 256) return (l << 10) | (1u << 15);
+  if (sym == 256) return 7u | (3u << 5) | (kStepEob << 15);
+  if (sym > 285) return u32(kBadSymbol) << 15;
+  const u32 x = length_extra(sym - 257);
+  return l | (x << 5) | ((l + x) << 10) | (length_base(sym - 257) << 15) | 0x80000000u;
+}
+__host__ __device__ __forceinline__ u32 fixed_step(u32 b, u32 entry) {
+  const u32 value = bit_field(entry, 15, 9) + bit_field(b, entry, entry >> 5);
+  const u32 lx = bit_field(entry, 10, 5);
+  const u32 d = __builtin_bitreverse32(b >> lx) >> 27;  // the distance symbol
+  const u32 follows = u32(i32(entry) >> 31);
+  const u32 half = d >> 1;
+  const u32 nb = lx + (((half > 1u ? half : 1u) + 4u) & follows);
+  return (d & follows) > 29 ? u32(kBadSymbol) << 6 : (nb << 1) | (value << 6);
+}
+// A step at bit p of a body that ends at bit `end`.
+__host__ __device__ __forceinline__ u32 fixed_step_within(u32 step, u32 p, u32 end) {
+  const u32 nb = (step & 63u) >> 1;
+  const bool eob = !nb && ((step >> 6) & kStepEob);
+  const u32 need = eob ? 7u : nb;  // of an error none
+  if (need && p + need > end) return u32(kTruncated) << 6;
+  return eob && p + 10 > end ? step | (8u << 6) : step;
+}
+
 // ---- wrapper formats -----------------------------------------------------------
 // zlib (RFC 1950), raw DEFLATE (RFC 1951 alone) and gzip (RFC 1952, one
 // member).  The drop-in zlib entry points use kFormatZlib without a

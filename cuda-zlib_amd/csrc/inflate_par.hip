@@ -2731,12 +2731,9 @@ __device__ __forceinline__ u64 wave_fetch_add(u64* p, u64 v) {
 
 // ---- one tile's decodes, by one workgroup ---------------------------------------
 // Every bit position of the tile is decoded once, independently (thread t: the
-// 32 positions from bit 32 t, out of registers), into a 16-bit step; the
+// 32 positions from bit 32 t, out of registers), into a 16-bit step (fixed_step); the
 // decodes of the 32 entries of each of the tile's 512-bit slices are then
 // chains of LDS reads over the steps, at most 73 long.
-//   step: twice the bits taken | the output bytes << 6 for a token; no bits for
-//   a special, whose value is kStepEob | the next header's three bits (| 8 if
-//   they are cut off) or an error's status.
 // Both parts are bound by VALU issue, so a position costs no branch and a link
 // of a chain four instructions (a first form, with branches and an unpacked
 // sum, took 1.7 times as long).
@@ -2745,16 +2742,11 @@ __device__ __forceinline__ u64 wave_fetch_add(u64* p, u64 v) {
 // token costs a thread of a nearly empty chip about 0.5 us), placing the
 // slices by one thread per tile 1210 us; this form 236 and 265 us.
 constexpr u32 kFixThreads = 256;
-constexpr u32 kStepEob = 16;
 static_assert(kFixThreads * 32 == kFixTileBits, "a thread decodes 32 positions");
 static_assert(kFixTileSlices * kFixEntries == 2 * kFixThreads, "two slice chains a thread");
 
 struct FixTileShared {
-  // Of the next 9 bits: where the length's extra bits start (bits 0-4), their
-  // number (5-9), the bits before a distance (10-14), the length's base
-  // (15-23), a distance follows (31).  An EOB takes the header's bits for
-  // extra ones.
-  u32 lut[512];
+  u32 lut[512];  // fixed_step_entry of the next 9 bits
   union {
     __align__(16) u16 step[kFixTileBits];
     FixSummary slice[kFixTileSlices][kFixEntries];  // of the slice's entries, relative to the tile
@@ -2762,30 +2754,7 @@ struct FixTileShared {
 };
 
 __device__ __forceinline__ void fix_build_lut(u32* lut) {
-  for (u32 i = threadIdx.x; i < 512; i += blockDim.x) {
-    const u32 r9 = __builtin_bitreverse32(i) >> 23;
-    u32 sym, l;
-    if ((r9 >> 2) < 24) {
-      sym = 256 + (r9 >> 2);
-      l = 7;
-    } else if ((r9 >> 1) < 0xC8) {
-      sym = (r9 >> 1) < 0xC0 ? (r9 >> 1) - 0x30 : (r9 >> 1) + 88;  // 0xC0 -> 280
-      l = 8;
-    } else {
-      sym = r9 - 256;
-      l = 9;
-    }
-    u32 v = (l << 10) | (1u << 15);  // a literal
-    if (sym == 256) {
-      v = 7u | (3u << 5) | (kStepEob << 15);
-    } else if (sym > 285) {
-      v = u32(kBadSymbol) << 15;
-    } else if (sym > 256) {
-      const u32 x = length_extra(sym - 257);
-      v = l | (x << 5) | ((l + x) << 10) | (length_base(sym - 257) << 15) | 0x80000000u;
-    }
-    lut[i] = v;
-  }
+  for (u32 i = threadIdx.x; i < 512; i += blockDim.x) lut[i] = fixed_step_entry(i);
 }
 
 // The steps of tile k's positions from bit 32 t.  `end`: the body's end
@@ -2808,21 +2777,8 @@ __device__ __forceinline__ void fix_steps(const u8* body, u64 len, u64 k, u32 en
     for (u32 j = 0; j < 8; ++j) {
       const u32 i = i8 + j;
       const u32 b = __builtin_amdgcn_alignbit(a1, a0, i);
-      const u32 v = lut[b & 511u];
-      const u32 value = __builtin_amdgcn_ubfe(v, 15, 9) + __builtin_amdgcn_ubfe(b, v, v >> 5);
-      const u32 lx = __builtin_amdgcn_ubfe(v, 10, 5);
-      const u32 d = __builtin_bitreverse32(b >> lx) >> 27;  // the distance symbol
-      const u32 follows = u32(i32(v) >> 31);
-      const u32 nb = lx + ((max(d >> 1, 1u) + 4u) & follows);
-      u32 r = (nb << 1) | (value << 6);
-      if ((d & follows) > 29) r = u32(kBadSymbol) << 6;
-      if (kEnd) {
-        const u32 p = 32 * t + i;
-        const bool eob = (r & 63u) == 0 && (value & kStepEob), token = (r & 63u) != 0;
-        if ((token && p + nb > end) || (eob && p + 7 > end)) r = u32(kTruncated) << 6;
-        else if (eob && p + 10 > end) r |= 8u << 6;
-      }
-      o[j] = r;
+      o[j] = fixed_step(b, lut[b & 511u]);
+      if (kEnd) o[j] = fixed_step_within(o[j], 32 * t + i, end);
     }
     *reinterpret_cast<uint4*>(step + 32 * t + i8) =
         make_uint4(o[0] | (o[1] << 16), o[2] | (o[3] << 16), o[4] | (o[5] << 16), o[6] | (o[7] << 16));
@@ -3066,16 +3022,15 @@ struct FixWalkShared {
   __align__(16) u16 step[kFixTileBits];
 };
 
-// An atomic add by lane 0, its old value given to every lane.
 }  // namespace
 
 // One wave per region: continue the paused segment from the fixed block at
 // its seg_end.  Every lane follows the same walk (uniform loads; lane 0
-// stores), and the wave loads summaries and stages tiles together.  Fixed
+// stores), and the wave loads summaries and decodes tiles together.  Fixed
 // runs are followed by summaries (a tile entered at a bit offset above 31, or
-// not marked, is decoded from the stage); stored blocks are parsed in place;
-// the segment ends at a final block, at a block boundary that is a candidate,
-// or at an error, as describe ends it.  Each finished run gets a block record
+// not marked, is decoded here); stored blocks are parsed in place; the segment
+// ends at a final block, at a block boundary that is a candidate, or at an
+// error, as describe ends it.  Each finished run gets a block record
 // (kRecFixedRun) with consecutive slice groups and a FixRun; each of its tiles
 // a FixTile slot for g_fix_slices.  When records, groups or slots run out the
 // segment keeps no records (serial emission).
@@ -5349,7 +5304,7 @@ __global__ __launch_bounds__(kRestThreads) void g_resolve_rest(const State* st, 
   hi = min<u64>(hi, lo + kRestBytes);
   if (lo >= hi) return;  // uniform
   const u64 g0 = lo >> kResolveGroupShift;
-  const u32 ng = u32((hi - lo + (1u << kResolveGroupShift) - 1) >> kResolveGroupShift);  // <= 16
+  const u32 ng = u32((hi - lo + (1u << kResolveGroupShift) - 1) >> kResolveGroupShift);  // <= 8
   const u32 marked = u32(__ballot(lane < ng && marks[g0 + lane]));
   if (!marked) return;  // uniform
   if (!t) listed = 0;

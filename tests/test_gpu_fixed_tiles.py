@@ -7,6 +7,7 @@ import zlib
 import numpy as np
 import pytest
 
+import deflate_writer as dw
 import workloads
 from oracle import oracle
 
@@ -161,3 +162,24 @@ def test_fixed_blocks_between_dynamic_ones(gpu, length, gap):
     stream = b"\x78\x9c" + body + zlib.adler32(raw).to_bytes(4, "big")
     assert zlib.decompress(stream) == raw
     _check(gpu, stream, raw, length % 4)
+
+
+@pytest.mark.parametrize("length", [3, 19, 58, 130, 257])
+@pytest.mark.parametrize("distance_code", [29, 30, 31])
+def test_run_that_ends_in_a_match(gpu, length, distance_code):
+    """A run's last bits are a match, with a distance code that stands for nothing or cut
+    short: the oracle's statuses at every cut."""
+    import cuda_zlib
+    raw = _content("text", 90000)
+    w = dw.BitWriter()
+    block = dw.Block(w, True).literals(raw)
+    li = max(i for i, base in enumerate(dw.LENGTH_BASE) if base <= length)
+    w.code(block.ll[257 + li]).put(length - dw.LENGTH_BASE[li], dw.LENGTH_EXTRA[li])
+    w.code((distance_code, 5))
+    body = w.getvalue()
+    for cut in range(4):
+        stream = dw.wrap(body[:len(body) - cut], raw)
+        want, status = oracle.decompress(stream, len(raw) + length)
+        out, meta = cuda_zlib.decompress_zlib_checked(stream, len(raw) + length, gpu)
+        assert status and int(meta.cpu().numpy()[0]) == status
+        assert out.cpu().numpy().tobytes() == want
