@@ -25,11 +25,29 @@ def _fixed(data, every=0):
     return out + c.flush()
 
 
+def _literal_run(data, final=True):
+    """One fixed block of literals only, as the bits it takes (zlib stores such data)."""
+    byte = np.frombuffer(data, np.uint8).astype(np.int64)
+    length = np.where(byte < 144, 8, 9)
+    code = np.where(byte < 144, byte + 0x30, byte + 256)  # 144 -> 0x190
+    bits = (code[:, None] >> (length[:, None] - 1 - np.arange(9))) & 1
+    literals = bits[np.arange(9) < length[:, None]]
+    return np.concatenate(([int(final), 1, 0], literals, np.zeros(7, np.int64))).astype(np.uint8)
+
+
+def _literal_stream(data):
+    body = np.packbits(_literal_run(data), bitorder="little").tobytes()
+    assert body[0] >> 1 & 3 == 1
+    stream = dw.wrap(body, data)
+    assert zlib.decompress(stream) == data
+    return stream
+
+
 def _content(kind, n):
     rng = np.random.default_rng(n + 17)
     if kind == "text":
         return workloads.text_like(n, rng)
-    if kind == "noise":  # 8- and 9-bit literals only
+    if kind == "noise":  # 8- and 9-bit literals only, for _literal_stream
         return rng.integers(0, 256, n, dtype=np.uint8).tobytes()
     return workloads.runs_segment(n, rng)  # nearly every token a match of 258
 
@@ -49,7 +67,9 @@ def _check(gpu, stream, raw, skew):
 @pytest.mark.parametrize("size", [66000, 70001, 131072, 140003, 1000003])
 def test_runs_of_every_length(gpu, kind, size):
     raw = _content(kind, size)
-    _check(gpu, _fixed(raw), raw, size % 4)
+    stream = _literal_stream(raw) if kind == "noise" else _fixed(raw)
+    assert stream[2] >> 1 & 3 == 1
+    _check(gpu, stream, raw, size % 4)
 
 
 @pytest.mark.parametrize("every", [150, 700, 1024, 1700, 66000, 120001])
@@ -58,20 +78,33 @@ def test_runs_that_start_and_end_inside_tiles(gpu, every):
     _check(gpu, _fixed(raw, every), raw, every % 4)
 
 
-@pytest.mark.parametrize("end", [1024, 2048, 64 * 1024, 128 * 1024])
-def test_runs_that_end_at_tile_and_group_edges(gpu, end):
-    """Streams cut by a byte at a time to end just before, at and after an edge
-    of the body (whose first byte is the stream's third)."""
-    import cuda_zlib
-    data = _content("noise", 2 * end)
-    for tail in range(-2, 4):
-        n = int((end + tail) * 8 / 8.44)
-        raw = data[:n]
-        stream = _fixed(raw)
-        raw = _content("noise", 70000) + raw  # past the small route, in one run
-        _check(gpu, _fixed(raw), raw, tail & 3)
-        out = cuda_zlib.decompress_zlib(stream, n, gpu)
-        assert out.cpu().numpy().tobytes() == raw[70000:]
+@pytest.mark.parametrize("start", [0, 3 * 1024 - 1, 3 * 1024, 3 * 1024 + 1, 64 * 1024])
+@pytest.mark.parametrize("end", [70 * 1024, 71 * 1024, 128 * 1024, 192 * 1024])
+def test_runs_that_end_at_tile_and_group_edges(gpu, start, end):
+    """Literal runs whose end of block lies bits before, at and after the edge of a tile
+    or a group, from byte `start` of the body on (behind stored blocks)."""
+    rng = np.random.default_rng(start + end)
+    prefix, before = b"", b""
+    while len(prefix) < start:
+        n = min(start - len(prefix) - 5, 60000)
+        if 0 < start - len(prefix) - 5 - n < 6:
+            n -= 6
+        piece = rng.integers(0, 256, n, dtype=np.uint8).tobytes()
+        prefix += dw.stored(piece, final=False)
+        before += piece
+    assert len(prefix) == start
+    for delta in (-17, -8, -1, 0, 1, 7, 8, 25):
+        bits = 8 * (end - start) + delta - 10  # of the literals
+        long = bits % 8 + 8 * (bits // 80)     # with 9-bit codes
+        short = (bits - 9 * long) // 8
+        data = np.concatenate((rng.integers(144, 256, long), rng.integers(0, 144, short)))
+        data = rng.permutation(data.astype(np.uint8)).tobytes()
+        run = _literal_run(data)
+        assert len(run) == 8 * (end - start) + delta
+        raw = before + data
+        stream = dw.wrap(prefix + np.packbits(run, bitorder="little").tobytes(), raw)
+        assert zlib.decompress(stream) == raw
+        _check(gpu, stream, raw, delta & 3)
 
 
 @pytest.mark.parametrize("keep", [0.02, 0.3, 0.77, 0.999])
