@@ -2689,12 +2689,27 @@ __global__ __launch_bounds__(kDescThreads) void g_describe(
 
 // Marks the tiles of every region for g_fix_sum: from the region's start to
 // the first later candidate whose own segment did not fail (header
-// look-alikes inside a run fail), at most kFixMarkScan candidates on.
-__global__ __launch_bounds__(256) void g_fix_mark(const State* st, const u64* cand, u64 len,
+// look-alikes inside a run fail), at most kFixMarkScan candidates on.  A
+// final block that ends before the body does (in an open-ended body, with no
+// member after its trailer) is a look-alike too: its codes are complete, so its
+// garbage decodes to some end of block.  (Taken for the run's end, the rest of
+// the run had no summaries and the walk decoded it tile by tile: 15 MiB of one
+// run 469 ms, now 1.8.)
+__global__ __launch_bounds__(256) void g_fix_mark(const u8* body, const State* st, const u64* cand,
+                                                  u64 len,
                                                   const u64* seg_end, const u32* seg_flags,
                                                   const u32* region_cand, u32* fix_need,
-                                                  u64 tiles) {
+                                                  u64 tiles, OpenEnd open) {
   if (st->status) return;
+  const auto stream_end = [&](u64 bit) {
+    const u64 at = (bit + 7) / 8;
+    if (!open.open) return at == len;
+    const u64 next = at + open.trailer;
+    if (next + 2 > len) return true;
+    const u32 b0 = body[next], b1 = body[next + 1];
+    return open.trailer == 8 ? b0 == 0x1f && b1 == 0x8b
+                             : (b0 & 15) == 8 && (b0 * 256 + b1) % 31 == 0;
+  };
   const u64 regions = st->fix_regions, n = st->candidates;
   for (u64 r = threadIdx.x; r < regions; r += blockDim.x) {
     const u32 c = region_cand[r];
@@ -2702,7 +2717,9 @@ __global__ __launch_bounds__(256) void g_fix_mark(const State* st, const u64* ca
     u64 j = lower_bound_from(cand, n, c + 1, x + 1);
     u64 h = len * 8;
     for (u32 k = 0; j < n; ++j, ++k) {
-      if (k == kFixMarkScan || (seg_flags[j] & 0xffffu) == 0) {
+      const u32 flags = seg_flags[j];
+      if (k == kFixMarkScan ||
+          ((flags & 0xffffu) == 0 && (!(flags >> 31) || stream_end(seg_end[j])))) {
         h = cand[j];
         break;
       }
@@ -4795,7 +4812,7 @@ __global__ __launch_bounds__(kDescThreads) void g_batch_wide(
 
 // Large batch files after resolution: Adler-32 of each decoded file against
 // its trailer; [0, 0] when it matches, else the file is flagged for the
-// serial decoder (so are all of them if a chain stayed unresolved).
+// serial decoder.
 __global__ __launch_bounds__(256) void g_batch_wide_finish(const BatchFile* files, const u32* list,
                                                            u32 n, const u8* out, const State* st,
                                                            const u32* wanted, u32* redo,
@@ -4869,7 +4886,7 @@ __global__ __launch_bounds__(256) void g_batch_wide_finish(const BatchFile* file
 // ---- resolve: stripes of the output, each by one workgroup --------------------
 // Measured on one MI355X, 64 MiB of text (47 million unresolved bytes): rounds
 // that followed every byte's roots through memory, waiting on L2 misses, took
-// 1740 us; the stripes (bound by VALU issue) 207 us, the windows 44 us and the
+// 1740 us; the stripes (bound by VALU issue) 194 us, the windows 47 us and the
 // rest 134 us.  512 stripes, two workgroups per CU: 226, 196 and 139 us (a byte
 // survives a tile's walk past the stripe's start with a share that halves
 // about every 33 KiB, so short stripes leave more).
@@ -5725,8 +5742,8 @@ hipError_t run_inflate_general(hipStream_t stream, Scratch& scratch, const u8* i
             rec_capacity, slice_entry, slice_off, group_link, group_capacity, tables,
             table_capacity, slots, hdr_d0, hdr_info, seg_last, region_cand);
   HZ_TRY(hipGetLastError());
-  HZ_LAUNCH(g_fix_mark, dim3(1), dim3(256), 0, stream, st, cand, len, seg_end, seg_flags,
-            region_cand, fix_need, tiles);
+  HZ_LAUNCH(g_fix_mark, dim3(1), dim3(256), 0, stream, body, st, cand, len, seg_end, seg_flags,
+            region_cand, fix_need, tiles, open);
   HZ_TRY(hipGetLastError());
 
   // Long fixed-Huffman runs deferred by describe (each launch returns at once

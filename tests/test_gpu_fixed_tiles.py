@@ -216,3 +216,47 @@ def test_run_that_ends_in_a_match(gpu, length, distance_code):
         out, meta = cuda_zlib.decompress_zlib_checked(stream, len(raw) + length, gpu)
         assert status and int(meta.cpu().numpy()[0]) == status
         assert out.cpu().numpy().tobytes() == want
+
+
+def _final_block_look_alike():
+    """The bits of a final dynamic block without output, made so that they also parse as
+    tokens of the fixed codes: 105, and three zeros that end the last token."""
+    lengths = [0 if s in (3, 5, 14) else 4 for s in range(19)]
+    code = dw.canonical(lengths)
+    w = dw.BitWriter().put(1, 1).put(2, 2).put(0, 5).put(0, 5).put(15, 4)
+    for s in dw.CL_ORDER:
+        w.put(lengths[s], 3)
+    w.code(code[18]).put(138 - 11, 7).code(code[18]).put(118 - 11, 7)  # 256 lengths of zero
+    w.code(code[1]).code(code[0]).put(0, 1)  # the end of block's code, no distances; that code
+    assert w.nbits == 105
+    return np.unpackbits(np.frombuffer(w.put(0, 3).getvalue(), np.uint8), bitorder="little")[:108]
+
+
+@pytest.mark.parametrize("members", [False, True])
+def test_final_block_look_alike_in_a_run(gpu, members):
+    """A run whose tokens hold what reads as a final dynamic block, complete: the run does
+    not end there.  (With the rest of it walked tile by tile, some 40 times as long.)"""
+    import cuda_zlib
+    import torch
+    rng = np.random.default_rng(23)
+    first, rest = (rng.integers(0, 256, n, dtype=np.uint8).tobytes() for n in (40000, 1500000))
+
+    def decode_ms(middle):
+        body = np.concatenate((_literal_run(first)[:-7], middle, _literal_run(rest)[3:]))
+        body = np.packbits(body.astype(np.uint8), bitorder="little").tobytes()
+        raw = zlib.decompress(body, -15)
+        assert len(raw) > 1540000
+        src = torch.from_numpy(np.frombuffer(dw.wrap(body, raw), np.uint8).copy()).to(gpu)
+        times = []
+        for _ in range(6):
+            start, stop = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            start.record()
+            out, meta = cuda_zlib.decompress_zlib_checked(src, len(raw), gpu, members=members)
+            stop.record()
+            torch.cuda.synchronize()
+            times.append(start.elapsed_time(stop))
+            assert int(meta.cpu().numpy()[0]) == 0 and out.cpu().numpy().tobytes() == raw
+        return min(times)
+
+    plain = decode_ms(_literal_run(b"middle")[3:-7])
+    assert decode_ms(_final_block_look_alike()) < 3 * plain
