@@ -235,7 +235,7 @@ def _final_block_look_alike():
 @pytest.mark.parametrize("members", [False, True])
 def test_final_block_look_alike_in_a_run(gpu, members):
     """A run whose tokens hold what reads as a final dynamic block, complete: the run does
-    not end there.  (With the rest of it walked tile by tile, some 40 times as long.)"""
+    not end there.  (With the rest of it walked tile by tile, 200 times as long.)"""
     import cuda_zlib
     import torch
     rng = np.random.default_rng(23)

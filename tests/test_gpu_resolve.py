@@ -79,8 +79,8 @@ def test_few_bytes_in_long_chains(gpu, size):
 
 
 def test_long_chains_cost_little(gpu):
-    """Records whose field is copied take less than twice the time of records without
-    one (4.5 times as long with every chain followed link by link)."""
+    """Records whose field is copied take less than 1.5 times the time of records without
+    one (1.12 times; 2.1 times with every chain followed link by link)."""
     import cuda_zlib
     import torch
 
@@ -97,8 +97,8 @@ def test_long_chains_cost_little(gpu):
             times.append(start.elapsed_time(stop))
         return min(times)
 
-    n = 16 << 20
-    assert decode_ms(_records(n, b"record")) < 2 * decode_ms(_records(n, b""))
+    n = 32 << 20
+    assert decode_ms(_records(n, b"record")) < 1.5 * decode_ms(_records(n, b""))
 
 
 @pytest.mark.parametrize("skew", [1, 2, 3])
